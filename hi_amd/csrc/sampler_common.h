@@ -737,13 +737,13 @@ __device__ __forceinline__ void sort_ranked(FinLds& fs, int n) {
   __syncthreads();
 }
 
-// Descending bitonic sort of the keys buf[0..n), n <= PER * NT, keys only
-// (zero pads them and sorts last; equal keys are equal values).  PER
-// consecutive elements per thread in registers: distances below PER inside
-// the thread, up to 32 * PER across the lanes of a wave (DPP, swizzle and
-// bpermute lane moves), 64 * PER and more through buf with barriers.  buf
-// has room for PER * NT keys; all of them are written.
-template <int PER>
+// Descending bitonic sort of the keys buf[0..n), n <= PER * NTH, keys only
+// (zero pads them and sorts last; equal keys are equal values), by NTH
+// threads.  PER consecutive elements per thread in registers: distances
+// below PER inside the thread, up to 32 * PER across the lanes of a wave
+// (DPP, swizzle and bpermute lane moves), 64 * PER and more through buf with
+// barriers.  buf has room for PER * NTH keys; all of them are written.
+template <int PER, int NTH = NT>
 __device__ __forceinline__ void block_sort_desc(uint64_t* buf, int n) {
   const int tid = threadIdx.x;
   uint64_t x[PER];
@@ -758,7 +758,7 @@ __device__ __forceinline__ void block_sort_desc(uint64_t* buf, int n) {
     v = keep_max ? hi : lo;
   };
   #pragma unroll
-  for (int k = 2; k <= PER * NT; k <<= 1) {
+  for (int k = 2; k <= PER * NTH; k <<= 1) {
     #pragma unroll
     for (int j = k >> 1; j > 0; j >>= 1) {
       if (j >= 64 * PER) {
@@ -1104,210 +1104,13 @@ __device__ __forceinline__ int rank_candidates(FinLds& fs, const SampleArgs& a, 
 // (top-k rows); defined with the wave folds below.
 __device__ __forceinline__ uint32_t draw_topk(FinLds& fs, const RowCfg& cfg, int k);
 
-// Serial f32 fold of a global float array in index order (Rust's Sum: a fold
-// from -0.0), by thread 0, staged through LDS tiles.  Valid in all threads.
-__device__ __forceinline__ float fold_global(FinLds& fs, const float* x, int n) {
-  float* tile = reinterpret_cast<float*>(fs.cbig);
-  float acc = -0.0f;  // meaningful in thread 0 only
-  for (int t0 = 0; t0 < n; t0 += kTileFloats) {
-    const int m = min(kTileFloats, n - t0);
-    __syncthreads();
-    for (int i = threadIdx.x; i < m; i += NT) tile[i] = x[t0 + i];
-    __syncthreads();
-    if (threadIdx.x == 0)
-      for (int i = 0; i < m; ++i) acc += tile[i];
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) fs.fval0 = acc;
-  __syncthreads();
-  const float r = fs.fval0;
-  __syncthreads();
-  return r;
-}
+}  // namespace hi_rocm
 
-// Bitonic sort of a global array (descending) by one workgroup.
-__device__ __forceinline__ void global_sort_desc(uint64_t* g, int n2) {
-  for (int k = 2; k <= n2; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int i = threadIdx.x; i < n2; i += NT) {
-        const int ixj = i ^ j;
-        if (ixj > i) {
-          const uint64_t x = g[i], y = g[ixj];
-          const bool desc = (i & k) == 0;
-          if (desc ? (x < y) : (x > y)) { g[i] = y; g[ixj] = x; }
-        }
-      }
-      __syncthreads();
-    }
-  }
-}
+#include "sampler_draw.h"
 
-// Rows without top-k (or with top_k > 1024): the distribution is re-read from
-// the workspace (ws_s holds the scaled logits).  Returns the token or
-// 0xffffffff for the argmax fallback.
-__device__ __forceinline__ uint32_t draw_wide(FinLds& fs, const SampleArgs& a, int row, const RowCfg& cfg,
-                              float M, float u) {
-  const int tid = threadIdx.x;
-  const int V = a.V;
-  const float* srow = a.ws_s + (int64_t)row * V;
-  float* wrow = a.ws_w + (int64_t)row * V;
-  uint64_t* list = a.ws_list + (int64_t)row * a.list_stride;
-  for (int b = tid; b < kBins; b += NT) { fs.hist[b] = 0u; fs.mass[b] = 0ull; }
-  __syncthreads();
-  for (int i = tid; i < V; i += NT) {
-    float w = exact_expf(srow[i] - M);
-    if (w < cfg.min_p) w = 0.f;
-    wrow[i] = w;
-    if (w > 0.f) {
-      const uint32_t b = __float_as_uint(w) >> 20;
-      atomicAdd(&fs.hist[b], 1u);
-      atomicAdd((unsigned long long*)&fs.mass[b], (unsigned long long)((double)w * 1099511627776.0));
-    }
-  }
-  __syncthreads();
-  const bool wide_k = cfg.cls == kTopK;
-  float total = 0.f;
-  if (!wide_k) {
-    total = fold_global(fs, wrow, V);  // gpu.rs:837: vocab-order sum
-    if (total <= 0.f || !finitef_(total)) return 0xffffffffu;
-  }
-  if (tid == 0) {
-    uint64_t all_mass = 0;
-    for (int b = 0; b < kBins; ++b) all_mass += fs.mass[b];
-    int bstar = 0;
-    if (wide_k) {
-      uint32_t c = 0;
-      for (int b = kBins - 1; b >= 0; --b) { c += fs.hist[b]; if (c >= (uint32_t)cfg.k_eff) { bstar = b; break; } }
-    } else if (cfg.cutoff < 1.f) {
-      // superset holding the nucleus with margin (verified below)
-      const double need = fmin(1.0, (double)cfg.cutoff + 0.02) * (double)all_mass;
-      uint64_t c = 0;
-      for (int b = kBins - 1; b >= 0; --b) { c += fs.mass[b]; if ((double)c >= need) { bstar = b; break; } }
-    }
-    fs.flag = (uint32_t)bstar;
-  }
-  __syncthreads();
-  int bstar = (int)fs.flag;
-  uint32_t tok = 0xffffffffu;
-  for (int attempt = 0; attempt < 2; ++attempt) {
-    __syncthreads();
-    if (tid == 0) {
-      uint32_t off = 0;
-      for (int b = kBins - 1; b >= 0; --b) {
-        fs.aux[b] = off;
-        if (b >= bstar) off += fs.hist[b];
-      }
-      fs.counter = off;
-    }
-    __syncthreads();
-    const int n_sup = (int)fs.counter;
-    for (int i = tid; i < V; i += NT) {
-      const float w = wrow[i];
-      if (w > 0.f) {
-        const int b = (int)(__float_as_uint(w) >> 20);
-        if (b >= bstar) list[atomicAdd(&fs.aux[b], 1u)] = rank_key(w, (uint32_t)i);
-      }
-    }
-    __syncthreads();
-    const int n2 = next_pow2(max(n_sup, 1));
-    for (int i = n_sup + tid; i < n2; i += NT) list[i] = 0ull;
-    __syncthreads();
-    global_sort_desc(list, n2);
-    if (tid == 0) {
-      int k = n_sup;
-      if (wide_k) {
-        k = min(cfg.k_eff, n_sup);  // zero-weight entries add nothing
-        float t = -0.0f;
-        for (int i = 0; i < k; ++i) t += rank_w(list[i]);
-        total = t;
-      }
-      uint32_t r = 0xffffffffu;
-      uint32_t flag = 1u;
-      if (total > 0.f && finitef_(total)) {
-        float cum_p = 0.f;
-        int m_end = 0;
-        bool reached = false;
-        for (int i = 0; i < k; ++i) {
-          m_end = i + 1;
-          cum_p += rank_w(list[i]) / total;
-          if (cfg.cutoff < 1.f && cum_p >= cfg.cutoff) { reached = true; break; }
-        }
-        if (!wide_k && !reached && bstar != 0) {
-          flag = 0xffffffffu;  // superset too small: retry with every positive weight
-        } else {
-          float ct = -0.0f;
-          for (int i = 0; i < m_end; ++i) ct += rank_w(list[i]);
-          if (m_end > 0 && ct > 0.f && finitef_(ct)) {
-            const float target = clamp_uniform(u) * ct;
-            float cum = 0.f;
-            int pick = m_end - 1;
-            for (int i = 0; i < m_end; ++i) {
-              cum += rank_w(list[i]);
-              if (target < cum) { pick = i; break; }
-            }
-            r = cand_idx(list[pick]);
-          }
-        }
-      }
-      fs.token = r;
-      fs.flag = flag;
-    }
-    __syncthreads();
-    if (fs.flag != 0xffffffffu) { tok = fs.token; break; }
-    bstar = 0;
-  }
-  return tok;
-}
+namespace hi_rocm {
 
-// Temperature-only rows: kernels.cu:7803-7867 with the exact weight function.
-// 256 contiguous chunks, one per thread of the (256-thread) workgroup.
-__device__ __forceinline__ uint32_t draw_temp_only(FinLds& fs, const SampleArgs& a, int row, float M, float u,
-                                   uint32_t argmax_fin) {
-  static_assert(NT == 256, "the reference's temperature-only path uses 256 chunks");
-  const int tid = threadIdx.x;
-  const int V = a.V;
-  const float* srow = a.ws_s + (int64_t)row * V;
-  const int chunk = (V + 255) / 256;
-  float* csum = fs.fa;
-  float* prefix = fs.fb;
-  {
-    const int start = tid * chunk, end = min(start + chunk, V);
-    float s = 0.f;
-    for (int i = start; i < end; ++i) s += exact_expf(srow[i] - M);
-    csum[tid] = s;
-  }
-  __syncthreads();
-  if (tid == 0) {
-    float acc = 0.f;
-    for (int j = 0; j < 256; ++j) { prefix[j] = acc; acc += csum[j]; }
-    fs.fval0 = acc;
-    fs.token = 0xffffffffu;
-  }
-  __syncthreads();
-  const float total = fs.fval0;
-  if (total <= 0.f || !finitef_(total)) return argmax_fin;
-  const float uu = finitef_(u) ? fminf(fmaxf(u, 0.f), 0.99999994f) : 0.f;
-  const float target = uu * total;
-  {
-    const int start = tid * chunk, end = min(start + chunk, V);
-    const float lo = prefix[tid];
-    const float hi = lo + csum[tid];
-    if (start < end && target >= lo && (target < hi || tid == 255)) {
-      float cum = lo;
-      int chosen = -1;
-      for (int i = start; i < end; ++i) {
-        const float w = exact_expf(srow[i] - M);
-        if (w <= 0.f) continue;
-        chosen = i;
-        cum += w;
-        if (target < cum) break;
-      }
-      if (chosen >= 0) atomicMin(&fs.token, (uint32_t)chosen);
-    }
-  }
-  __syncthreads();
-  return fs.token != 0xffffffffu ? fs.token : argmax_fin;
-}
+static_assert(sizeof(DrawLds<NT>) <= sizeof(FinLds), "the draws reuse the finish's LDS");
 
 // argmax_host (gpu.rs:739-751, total_cmp, lowest index) over the processed
 // logits of the row.  Only needed when no scaled logit is finite (or l / T
@@ -1429,9 +1232,11 @@ __device__ __forceinline__ void finish_row(FinLds& fs, const SampleArgs& a, int 
     token = pick < 0 ? 0xffffffffu : cand_idx(fs.buf[pick]);
     if (token == 0xffffffffu) token = row_argmax_total(fs, a, row, cfg);
   } else if (cfg.cls == kTempOnly) {
-    token = draw_temp_only(fs, a, row, M, u, am_fin);
+    __syncthreads();
+    token = draw_temperature<NT>(reinterpret_cast<DrawLds<NT>&>(fs), a, row, M, u, am_fin);
   } else {
-    token = draw_wide(fs, a, row, cfg, M, u);
+    __syncthreads();
+    token = draw_ranked<NT>(reinterpret_cast<DrawLds<NT>&>(fs), a, row, cfg, M);
     if (token == 0xffffffffu) token = row_argmax_total(fs, a, row, cfg);
   }
   if (tid == 0) a.out_tokens[row] = token;

@@ -315,9 +315,7 @@ __device__ __forceinline__ uint64_t wave_select(const Segs<NS>& sg, uint32_t nee
 
 // Range-checked loads of one row (byte offsets at or past the range read
 // as zero; nothing faults).
-typedef int i32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x2_t __attribute__((ext_vector_type(2)));
-constexpr int kBufferConfig = 0x00020000;  // raw buffer, 32-bit data (gfx9 family)
 
 struct RowBuf {
   __amdgpu_buffer_rsrc_t logits, mask;

@@ -5,6 +5,10 @@
 
 namespace hi_rocm {
 
+// Range-checked buffer accesses.
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
+constexpr int kBufferConfig = 0x00020000;  // raw buffer, 32-bit data (gfx9 family)
+
 // DPP controls (gfx9 encodings)
 constexpr int kDppXor1 = 0xB1;         // quad_perm [1,0,3,2]
 constexpr int kDppXor2 = 0x4E;         // quad_perm [2,3,0,1]
