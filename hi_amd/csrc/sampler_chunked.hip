@@ -49,42 +49,59 @@ __global__ void __launch_bounds__(NT) finish_kernel(SampleArgs a) {
   finish_row(fs, a, row, cfg);
 }
 
-// the rest chunks 1 .. of each row in turn.  Top-p rows take the wide pass
-// on every chunk; every other row is finished by its chunk-0 workgroup
-// (finish_lean, else finish_row) and its other workgroups exit at once.
-// Workgroups go to the XCDs and their shader engines round-robin by linear
-// id, so the B finishing workgroups, being consecutive, spread over the
-// whole chip (on a (chunks, rows) grid they would share a few engines).
-__global__ void __launch_bounds__(NT) finish_grid_kernel(SampleArgs a) {
+// Workgroups 0 .. B - 1 are the rows' unit 0, the rest units 1 .. of each row
+// in turn.  Top-p and temperature-only rows take the wide pass on every
+// unit; every other row is finished by its unit-0 workgroup (finish_lean,
+// else finish_row) and its other workgroups exit at once.  Workgroups go to
+// the XCDs and their shader engines round-robin by linear id, so the B
+// finishing workgroups, being consecutive, spread over the whole chip (on a
+// (chunks, rows) grid they would share a few engines).
+__global__ void __launch_bounds__(NT) finish_grid_kernel(SampleArgs a, WideUnits wu) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  int row = (int)blockIdx.x, chunk = 0;
+  int row = (int)blockIdx.x, unit = 0;
   if (row >= a.B) {
-    const int rest = row - a.B, per = a.n_chunks - 1;
+    const int rest = row - a.B, per = wu.n - 1;
     row = rest / per;
-    chunk = 1 + rest % per;
+    unit = 1 + rest % per;
   }
   const RowCfg cfg = load_cfg(a.pv, row, a.V, a.n_lp, a.need_lse);
-  if (cfg.cls != kTopP) {
-    if (chunk != 0) return;
-    FinLds& fs = *reinterpret_cast<FinLds*>(lds_raw);
+  FinLds& fs = *reinterpret_cast<FinLds*>(lds_raw);
+  // (the reference chunks' sums of a temperature-only row need 256 floats of
+  // its ws_list)
+  const bool wide = wide_fits(a) &&
+                    (cfg.cls == kTopP || (cfg.cls == kTempOnly && a.list_stride >= 128 && wu.n >= kTempSplit && a.B <= kTempRows));
+  if (!wide) {
+    if (unit != 0) return;
     if (finish_lean(fs, a, row, cfg)) return;
     __syncthreads();
     finish_row(fs, a, row, cfg);
     return;
   }
+  const int parts = cfg.cls == kTopP ? wu.n : kTempSplit;  // workgroups of the row that work
+  if (unit >= parts) return;
   WideChunkLds& L = *reinterpret_cast<WideChunkLds*>(lds_raw);
-  float pre[kWidePre];
-  const WideRowStats st = wide_row_stats(L, a, row, chunk, cfg, pre);
-  const bool valid = st.valid != 0u;
-  const float M = st.M, w_lo = st.w_lo;
-  if (valid) wide_chunk_work(L, lds_raw, a, row, chunk, cfg, M, w_lo, st.pred, st.mass, pre);
+  const DrawRow r = draw_row<NT>(a, row);
+  bool valid;
+  float M, w_lo = 0.f;
+  if (cfg.cls == kTopP) {
+    i32x4_t pre[kWidePre][4];
+    const WideRowStats st = wide_row_stats(L, a, row, wu, unit, cfg, r, pre);
+    valid = st.valid != 0u;
+    M = st.M;
+    w_lo = st.w_lo;
+    if (valid) wide_chunk_work(L, a, row, wu, unit, cfg, r, M, w_lo, st.pred, pre);
+  } else {
+    M = wide_row_max(a, row, cfg, L.wcnt);
+    valid = finitef_(M);
+    if (valid) wide_temperature_work(L, a, row, unit, r, M);
+  }
   // the last workgroup of the row finishes it (as select_finish_kernel)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
   uint32_t* counter = a.done + row;
   if (threadIdx.x == 0) {
     __threadfence();
-    L.last = atomicAdd(counter, 1u) == (uint32_t)(a.n_chunks - 1) ? 1u : 0u;
+    L.last = atomicAdd(counter, 1u) == (uint32_t)(parts - 1) ? 1u : 0u;
     if (L.last) {
       __threadfence();
       *counter = 0u;
@@ -92,15 +109,27 @@ __global__ void __launch_bounds__(NT) finish_grid_kernel(SampleArgs a) {
   }
   __syncthreads();
   if (L.last == 0u) return;
-  // every workgroup of the row has read the chunks' statistics: clear their
-  // valid flags, so that a chunk the next call's pass does not write is seen
-  for (int c = threadIdx.x; c < a.n_chunks; c += NT) a.wstat[(int64_t)row * a.n_chunks + c].valid = 0u;
-  uint32_t token = 0xffffffffu;
-  uint32_t path = kWideNoStats;
-  if (valid) token = wide_finish(lds_raw, a, row, cfg, M, w_lo, path);
-  if (threadIdx.x == 0) a.diag[row] = path;
   __syncthreads();
-  FinLds& fs = *reinterpret_cast<FinLds*>(lds_raw);
+  DrawLds<NT>& D = *reinterpret_cast<DrawLds<NT>*>(lds_raw);
+  uint32_t token = 0xffffffffu;
+  if (cfg.cls == kTempOnly) {
+    if (!valid) {
+      finish_row(fs, a, row, cfg);
+      return;
+    }
+    D.u.to.csum[threadIdx.x] = reinterpret_cast<const float*>(a.ws_list + (int64_t)row * a.list_stride)[threadIdx.x];
+    if (threadIdx.x < 32) D.exptab[threadIdx.x] = exp2_tab32(threadIdx.x);
+    __syncthreads();
+    token = draw_chunk_pick<NT>(D, r, M, cfg.u, 0xffffffffu);
+  } else {
+    // every workgroup of the row has read the chunks' statistics: clear their
+    // valid flags, so that a chunk the next call's pass does not write is seen
+    for (int c = threadIdx.x; c < a.n_chunks; c += NT) a.wstat[(int64_t)row * a.n_chunks + c].valid = 0u;
+    uint32_t path = kWideNoStats;
+    if (valid) token = wide_finish(D, a, row, cfg, wu, r, w_lo, path);
+    if (threadIdx.x == 0) a.diag[row] = path;
+  }
+  __syncthreads();
   if (token == 0xffffffffu) {
     finish_row(fs, a, row, cfg);
     return;
@@ -109,10 +138,9 @@ __global__ void __launch_bounds__(NT) finish_grid_kernel(SampleArgs a) {
   if (a.n_lp > 0 || a.out_token_lp) finish_logprobs(fs, a, row, cfg, token, M, false, 0);
 }
 
-size_t finish_grid_lds(int chunk) {
-  size_t b = sizeof(FinLds);
-  b = b > wide_chunk_lds(chunk) ? b : wide_chunk_lds(chunk);
-  b = b > wide_fin_lds(chunk) ? b : wide_fin_lds(chunk);
+size_t finish_grid_lds() {
+  size_t b = sizeof(FinLds) > sizeof(WideChunkLds) ? sizeof(FinLds) : sizeof(WideChunkLds);
+  b = b > sizeof(WideRunLds) ? b : sizeof(WideRunLds);
   return (b + 15) & ~(size_t)15;
 }
 
@@ -188,12 +216,13 @@ hipError_t launch_sample(const SampleArgs& a, hipStream_t stream, const LaunchEv
   e = launch_select(a, stream);
   if (e == hipSuccess) e = record(le, 1, stream);
   if (e != hipSuccess) return e;
-  const int64_t n_wg = (int64_t)a.n_chunks * a.B;
+  const WideUnits wu = wide_units(a.B, a.V, a.chunk, a.n_chunks);
+  const int64_t n_wg = (int64_t)wu.n * a.B;
   if (n_wg * NT >= ((int64_t)1 << 32)) return hipErrorInvalidConfiguration;  // 1-D grid of work-items
-  const size_t lds = finish_grid_lds(a.chunk);
+  const size_t lds = finish_grid_lds();
   e = ensure_lds((const void*)finish_grid_kernel, lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(finish_grid_kernel, dim3((unsigned)n_wg), dim3(NT), lds, stream, a);
+  hipLaunchKernelGGL(finish_grid_kernel, dim3((unsigned)n_wg), dim3(NT), lds, stream, a, wu);
   e = hipGetLastError();
   return e == hipSuccess ? record(le, 2, stream) : e;
 }

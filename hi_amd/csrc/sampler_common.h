@@ -19,7 +19,7 @@
 //                       finish_grid_kernel on a 1-D grid whose first B
 //                       workgroups finish the rows (spread over every XCD)
 //                       and whose other workgroups run the wide pass of
-//                       top-p rows.
+//                       top-p and temperature-only rows.
 //   scan + finish       more than 256 logprobs, or rows not aligned for
 //                       vector loads: scan_generic_kernel, then
 //                       finish_kernel, one workgroup per row.
@@ -32,13 +32,12 @@
 // Finishes: the lean finish (greedy; top-k <= 256) ranks by counting and
 // runs the reference's sequential f32 folds on every wave from registers
 // (wave_draw); top-k rows up to 1024 rank their candidates (register
-// bitonic sort) and draw the same way; top-p rows without top-k take the
-// wide pass: exact weights per chunk, the vocabulary-order normaliser as an
-// exact parallel emulation of the f32 fold (exact_fold.h / fold_wg.h: per
-// binade integer maps, one real add per binade crossing), the nucleus from
-// a mass histogram as a superset of distinct weights, and the rank-order
-// folds over those runs in closed form.  finish_row is the general
-// fallback and reproduces the reference step by step.
+// bitonic sort) and draw the same way; rows that need their whole
+// distribution (top-p without top-k, min-p alone, temperature only, top-k
+// above 1024) fold it exactly in parallel (sampler_draw.h), by one workgroup
+// or, on larger grids, by one per part of the row (sampler_wide.h).
+// finish_row is the general fallback and reproduces the reference step by
+// step.
 //
 // Every operation that decides a token mirrors the reference bit for bit
 // (crates/hi-cuda/src/gpu.rs:753-900): IEEE f32 division and addition in

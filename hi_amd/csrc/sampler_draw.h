@@ -44,6 +44,7 @@ constexpr int kDrawPiece = 4096;  // weights sorted at a time
 constexpr int kDrawBlocks = 256;  // blocks of a piece in its folds
 constexpr int kDrawDigitBits = 9;
 constexpr int kDrawDigits = 1 << kDrawDigitBits;  // of a radix pass
+constexpr int kDrawChunks = 256;  // chunks of a row whose lists a draw reads
 constexpr int kDrawRecs = 64;     // pieces whose start the draw can go back to
 constexpr uint32_t kOneBits = 0x3f800000u;
 
@@ -74,10 +75,11 @@ struct DrawLds {
   uint32_t hist[kDrawBins + kDrawBins / 32 + 64];  // (past the bins: a word per lane that nothing reads)
   fold::Map tmap[kDrawTiles], tlow[kDrawTiles];  // a tile's map in binade tbin, and in tbin - 1
   float tsum[kDrawTiles];
-  uint32_t tbin[kDrawTiles];  // bits 0-8: predicted binade; bit 9: tlow is there; 0: fold it exactly
+  uint32_t tbin[kDrawTiles];  // draw_tile_bin
   uint64_t exptab[32];
   uint64_t rec_hi[kDrawRecs];
   float rec_ct[kDrawRecs];
+  uint32_t noff[kDrawChunks + 1];  // a list's entries before each chunk
   uint32_t red[NTH / 64];
   uint64_t lo;
   uint32_t n, bnext, token;
@@ -259,7 +261,24 @@ __device__ __forceinline__ void draw_weights(DrawLds<NTH>& D, const DrawRow& r, 
   __syncthreads();
 }
 
-// Predicted binades of the tiles (wave 0), from a scan of their sums.
+// The binade a tile predicted to go from S to E is mapped in (bits 0-8; 0:
+// it is folded exactly), and whether the binade below is mapped too (bit 9).
+// A tile without a positive weight (min-p and masks leave many) adds nothing
+// in any binade.
+constexpr uint32_t kTileLow = 512u, kTileZero = 1024u;
+__device__ __forceinline__ uint32_t draw_tile_bin(double S, float sum) {
+  if (sum == 0.f) return kTileZero;
+  const double E = S + (double)sum;
+  const int e = fold::binade((float)S);
+  // well inside one binade (0.1%)
+  const bool one = e > 1 && fold::binade((float)(S * 0.999)) == e && fold::binade((float)(E * 1.001)) == e;
+  // terms below half an ulp add nothing to an f32 sum: the sum may lag the
+  // prediction, so near a binade's lower end the one below is kept too
+  const bool low = e > 2 && fold::binade((float)(S * 0.875)) != e;
+  return one || low ? (uint32_t)e | (low ? kTileLow : 0u) : 0u;
+}
+
+// Predicted binades of the tiles (one wave), from a scan of their sums.
 template <int NTH>
 __device__ __forceinline__ void draw_predict(DrawLds<NTH>& D, int nt) {
   const int lane = (int)(threadIdx.x & 63u);
@@ -267,19 +286,26 @@ __device__ __forceinline__ void draw_predict(DrawLds<NTH>& D, int nt) {
   double before = 0.0;
   for (int tb = 0; tb < nt; tb += 64) {
     const int t = tb + lane;
-    const double v = t < nt ? (double)D.tsum[t] : 0.0;
-    const double inc = fold::wave_scan_f64(v);
-    const double S = before + inc - v, E = before + inc;
-    const int e = fold::binade((float)S);
-    // a tile predicted to start and end well inside one binade (0.1%)
-    const bool one = e > 1 && fold::binade((float)(S * 0.999)) == e && fold::binade((float)(E * 1.001)) == e;
-    // terms below half an ulp add nothing to an f32 sum: the sum may lag
-    // the prediction, so near a binade's lower end the one below is kept too
-    const bool low = e > 2 && fold::binade((float)(S * 0.875)) != e;
-    if (t < nt) D.tbin[t] = one || low ? (uint32_t)e | (low ? 512u : 0u) : 0u;
+    const float s = t < nt ? D.tsum[t] : 0.f;
+    const double inc = fold::wave_scan_f64((double)s);
+    if (t < nt) D.tbin[t] = draw_tile_bin(before + inc - (double)s, s);
     const uint64_t ib = readlane64((uint64_t)__double_as_longlong(inc), 63);
     before += __longlong_as_double((long long)ib);
   }
+}
+
+// The maps of a tile's step (lane l's terms x) in its binade and, when kept,
+// in the one below: the composition over the lanes, in every lane.
+__device__ __forceinline__ void draw_tile_map(const float (&x)[kDrawPer], uint32_t bin, fold::Map& m, fold::Map& low) {
+  const int e = (int)(bin & 511u);
+  auto total_of = [&](fold::Map lm) {
+    const fold::Map inc = fold::wave_map_scan(lm);
+    return fold::Map{(uint32_t)__builtin_amdgcn_readlane((int)inc.t0, 63),
+                     (uint32_t)__builtin_amdgcn_readlane((int)inc.t1, 63)};
+  };
+  m = total_of(lane_map(x, e));
+  low = fold::map_identity();
+  if (bin & kTileLow) low = total_of(lane_map(x, e - 1));
 }
 
 // A tile's lane blocks of 16 terms (lane l: terms c0 + 16 l ..), straight
@@ -345,6 +371,44 @@ __device__ __forceinline__ void draw_collect(DrawLds<NTH>& D, const float* tr, c
     if (at < (uint32_t)kDrawPiece) D.u.p.key0[at] = top - __float_as_uint(tr[lane * kTrLd + __ffs((int)mk) - 1]);
 }
 
+// The chain over the row's tiles from -0.0 (wave 0, lane l holding tile tb +
+// l), to D.total: scans over the tiles of one binade, exact folds of the
+// others.
+template <int NTH>
+__device__ __forceinline__ void draw_chain(DrawLds<NTH>& D, const DrawRow& r, int nt) {
+  const int lane = (int)(threadIdx.x & 63u);
+  const int span = 64 * kDrawPer * r.mult;
+  float acc = -0.0f;
+  for (int tb = 0; tb < nt; tb += 64) {
+    const int n = min(64, nt - tb);
+    const uint32_t bin = lane < n ? D.tbin[tb + lane] : 0u;
+    const fold::Map mh = D.tmap[min(tb + lane, nt - 1)], ml = D.tlow[min(tb + lane, nt - 1)];
+    int i0 = 0;
+    while (i0 < n) {
+      const int e = fold::binade(acc);
+      const uint32_t A = fold::to_A(acc), p = A & 1u;
+      const int d = (int)(bin & 511u) - e;
+      fold::Map s = d == 0 ? mh : ml;
+      if (!(d == 0 || (d == 1 && (bin & kTileLow)))) s = fold::Map{fold::kSat, fold::kSat};
+      if (lane < i0 || bin == kTileZero) s = fold::map_identity();
+      const fold::Map inc = fold::wave_map_scan(s);
+      const uint32_t Ai = A + fold::apply(inc, p);
+      const uint64_t bad = __ballot(lane >= i0 && lane < n && Ai >= fold::kTop);
+      const int f = bad ? __ffsll((unsigned long long)bad) - 1 : n;
+      if (f > i0) acc = fold::from_A((uint32_t)__builtin_amdgcn_readlane((int)Ai, f - 1), e);
+      if (f < n) {
+        for (int g = 0; g < r.mult; ++g) {
+          float x[kDrawPer];
+          draw_lane_terms(r, (tb + f) * span + g * 64 * kDrawPer, x);
+          acc = wave_fold_blocks(x, acc, [](float) {});
+        }
+      }
+      i0 = f + 1;
+    }
+  }
+  if (lane == 0) D.total = acc;
+}
+
 // Step 2: the vocabulary-order fold of the row's weights from -0.0, in
 // D.total, and the first piece [lo, hi)'s sort keys, gathered by the same
 // pass.  All threads call it (D.tbin and the range are known, D.n is 0).
@@ -362,55 +426,19 @@ __device__ __forceinline__ void draw_total(DrawLds<NTH>& D, const DrawRow& r, ui
     draw_turn(tr, v, x);
     draw_collect<NTH>(D, tr, x, c0, lo, hi, top);
     const uint32_t tb = t < nt ? D.tbin[t] : 0u;
-    if (tb == 0u) return;
-    const int e = (int)(tb & 511u);
+    if ((tb & 511u) == 0u) return;
     if (g == 0) m = low = fold::map_identity();
-    auto total_of = [&](fold::Map lm) {
-      const fold::Map inc = fold::wave_map_scan(lm);
-      return fold::Map{(uint32_t)__builtin_amdgcn_readlane((int)inc.t0, 63),
-                       (uint32_t)__builtin_amdgcn_readlane((int)inc.t1, 63)};
-    };
-    m = fold::compose(m, total_of(lane_map(x, e)));
-    if (tb & 512u) low = fold::compose(low, total_of(lane_map(x, e - 1)));
+    fold::Map sm, sl;
+    draw_tile_map(x, tb, sm, sl);
+    m = fold::compose(m, sm);
+    low = fold::compose(low, sl);
     if (g == r.mult - 1 && lane == 0) {
       D.tmap[t] = m;
       D.tlow[t] = low;
     }
   });
   __syncthreads();
-  // the chain (wave 0, lane l holding tile tb + l): scans over the tiles of
-  // one binade, exact folds of the others
-  if (wid == 0) {
-    float acc = -0.0f;
-    for (int tb = 0; tb < nt; tb += 64) {
-      const int n = min(64, nt - tb);
-      const uint32_t bin = lane < n ? D.tbin[tb + lane] : 0u;
-      const fold::Map mh = D.tmap[min(tb + lane, nt - 1)], ml = D.tlow[min(tb + lane, nt - 1)];
-      int i0 = 0;
-      while (i0 < n) {
-        const int e = fold::binade(acc);
-        const uint32_t A = fold::to_A(acc), p = A & 1u;
-        const int d = (int)(bin & 511u) - e;
-        fold::Map s = d == 0 ? mh : ml;
-        if (bin == 0u || !(d == 0 || (d == 1 && (bin & 512u)))) s = fold::Map{fold::kSat, fold::kSat};
-        if (lane < i0) s = fold::map_identity();
-        const fold::Map inc = fold::wave_map_scan(s);
-        const uint32_t Ai = A + fold::apply(inc, p);
-        const uint64_t bad = __ballot(lane >= i0 && lane < n && Ai >= fold::kTop);
-        const int f = bad ? __ffsll((unsigned long long)bad) - 1 : n;
-        if (f > i0) acc = fold::from_A((uint32_t)__builtin_amdgcn_readlane((int)Ai, f - 1), e);
-        if (f < n) {
-          for (int g = 0; g < r.mult; ++g) {
-            float x[kDrawPer];
-            draw_lane_terms(r, (tb + f) * span + g * 64 * kDrawPer, x);
-            acc = wave_fold_blocks(x, acc, [](float) {});
-          }
-        }
-        i0 = f + 1;
-      }
-    }
-    if (lane == 0) D.total = acc;
-  }
+  if (wid == 0) draw_chain<NTH>(D, r, nt);
   __syncthreads();
 }
 
@@ -665,26 +693,6 @@ __device__ __forceinline__ void draw_gather(DrawLds<NTH>& D, const DrawRow& r, u
   __syncthreads();
 }
 
-// The next piece below hi, in rank order in D.wf(): its smallest key in lo,
-// its length returned, `bin` advanced to the histogram bin after it (~0u
-// once pieces come from the descent).  All threads call it.
-template <int NTH>
-__device__ __forceinline__ int draw_piece(DrawLds<NTH>& D, const DrawRow& r, uint64_t hi, uint64_t& lo, uint32_t& bin) {
-  if (bin != 0xffffffffu) {
-    __syncthreads();
-    if (threadIdx.x < 64) draw_bins<NTH>(D, bin, __builtin_inff());
-    __syncthreads();
-    bin = D.bnext;
-    lo = D.lo;
-  }
-  if (bin == 0xffffffffu) {
-    draw_descend<NTH>(D, r, hi);
-    lo = D.lo;
-  }
-  draw_gather<NTH>(D, r, lo, hi);
-  return draw_sort<NTH>(D, lo, hi);
-}
-
 // The ord-th (from 0) smallest index among the row's weights equal to w with
 // keys in [lo, hi).  All threads call it.
 template <int NTH>
@@ -781,77 +789,66 @@ __device__ __forceinline__ uint32_t draw_block_min(DrawLds<NTH>& D, uint32_t v) 
   return ~block_max_u32<NTH>(~v, D.red);
 }
 
-// The whole draw (gpu.rs:820-899) for a top-p row, or a top-k row of more
-// than kBuf ranks.  Returns the token, or 0xffffffff for the argmax
-// fallback.  All threads call it.
+// Where the ranks' weights come from: the row's weights in ws_w.
 template <int NTH>
-__device__ __forceinline__ uint32_t draw_ranked(DrawLds<NTH>& D, const SampleArgs& a, int row, const RowCfg& cfg,
-                                                float M) {
-  const int tid = threadIdx.x;
-  const DrawRow r = draw_row<NTH>(a, row);
-  const int span = 64 * kDrawPer * r.mult;
-  const int nt = (r.V + span - 1) / span;
-  draw_weights<NTH>(D, r, M, cfg.min_p);
-  const int k = cfg.cls == kTopK ? cfg.k_eff : 0;
-  const bool cut = cfg.cutoff < 1.f;
-  constexpr uint64_t kAll = ((uint64_t)kOneBits + 1u) << 23;
-  constexpr uint64_t kEnd = 1ull << 23;  // no positive weight has a smaller key
-  // pieces: keys [lo, hi), bin: the histogram bin after them (~0u: a descent
-  // overwrote the histogram, later pieces descend too)
-  uint64_t hi = kAll, lo;
-  uint32_t bin;
-  int n;
-  bool ready = false;  // the first piece is gathered
-  float total;
-  if (k == 0) {
-    // the first piece: the bins of the nucleus by their mass (within 0.8%)
-    if (tid >= 64 && tid < 128) draw_predict<NTH>(D, nt);
-    if (tid < 64) {
-      float s = 0.f;
-      for (int t = tid; t < nt; t += 64) s += D.tsum[t];
-      draw_bins<NTH>(D, 0u, cut ? (cfg.cutoff * 1.008f + 0.002f) * wave_sum_f32(s) : __builtin_inff());
-    }
-    if (tid == 0) D.n = 0u;
+struct DrawRowSrc {
+  const DrawRow& r;
+  bool whole;  // holds every positive weight of the row
+  __device__ __forceinline__ void gather(DrawLds<NTH>& D, uint64_t lo, uint64_t hi) const { draw_gather<NTH>(D, r, lo, hi); }
+  __device__ __forceinline__ bool descend(DrawLds<NTH>& D, uint64_t hi) const {
+    draw_descend<NTH>(D, r, hi);
+    return true;
+  }
+  __device__ __forceinline__ uint32_t index(DrawLds<NTH>& D, float w, uint32_t ord, uint64_t lo, uint64_t hi) const {
+    return draw_index<NTH>(D, r, w, ord, lo, hi);
+  }
+};
+
+// The next piece below hi, in rank order in D.wf(): its smallest key in lo,
+// its length returned, `bin` advanced to the histogram bin after it (~0u
+// once pieces come from the descent).  -1: the source cannot give it.  All
+// threads call it.
+template <int NTH, typename Src>
+__device__ __forceinline__ int draw_piece(DrawLds<NTH>& D, const Src& src, uint64_t hi, uint64_t& lo, uint32_t& bin) {
+  if (bin != 0xffffffffu) {
+    __syncthreads();
+    if (threadIdx.x < 64) draw_bins<NTH>(D, bin, __builtin_inff());
     __syncthreads();
     bin = D.bnext;
     lo = D.lo;
-    // (no first piece by the histogram: gather nothing)
-    draw_total<NTH>(D, r, bin != 0xffffffffu ? lo : kAll, hi);
-    total = D.total;
-    ready = bin != 0xffffffffu;
-  } else {
-    // the normaliser of the top k, in rank order
-    float t = -0.0f;
-    int seen = 0;
-    bin = 0u;
-    while (true) {
-      n = draw_piece<NTH>(D, r, hi, lo, bin);
-      draw_folds<NTH>(D, n, min(n, k - seen), 1.f, 0.f, t);
-      t = D.end[1];
-      seen += n;
-      if (seen >= k || lo <= kEnd || bin == (uint32_t)kDrawBins) break;
-      hi = lo;
-    }
-    if (bin != 0xffffffffu) bin = 0u;  // from the top again
-    hi = kAll;
-    total = t;
   }
-  __syncthreads();
-  if (!(total > 0.f) || !finitef_(total)) return 0xffffffffu;
+  if (bin == 0xffffffffu) {
+    if (!src.descend(D, hi)) return -1;
+    lo = D.lo;
+  }
+  src.gather(D, lo, hi);
+  return draw_sort<NTH>(D, lo, hi);
+}
 
-  // cum_p to the cutoff and the candidate total
+constexpr uint64_t kDrawAll = ((uint64_t)kOneBits + 1u) << 23;  // above every key
+constexpr uint64_t kDrawEnd = 1ull << 23;                       // no positive weight has a smaller key
+constexpr uint32_t kDrawFallback = 0xffffffffu;                 // the argmax fallback
+constexpr uint32_t kDrawRetry = 0xfffffffeu;                    // the source does not hold the nucleus
+
+// Step 3, from the normaliser `total`: ranks until the cutoff (or k ranks,
+// k > 0), the candidate total (also in *ct_out), the drawn index.  ready:
+// the first piece [lo, kDrawAll) is gathered and `bin` is the bin after it.
+// All threads call it.
+template <int NTH, typename Src>
+__device__ __forceinline__ uint32_t draw_ranks(DrawLds<NTH>& D, const Src& src, const RowCfg& cfg, int k, float total,
+                                               bool ready, uint64_t lo, uint32_t bin, float* ct_out) {
+  const int tid = threadIdx.x;
+  const bool cut = cfg.cutoff < 1.f;
   const float* wf = D.wf();
+  uint64_t hi = kDrawAll;
   float cum = 0.f, ct = -0.0f;
   int seen = 0, nrec = 0;  // ranks of the pieces before this one
-  int cnt;                 // candidates of the last piece
+  int n, cnt;              // the piece's ranks, and the candidates among the last one's
   float ct0;               // the candidate total before it
   while (true) {
-    if (ready) {
-      n = draw_sort<NTH>(D, lo, hi);
-    } else {
-      n = draw_piece<NTH>(D, r, hi, lo, bin);
-    }
+    n = ready ? draw_sort<NTH>(D, lo, hi) : draw_piece<NTH>(D, src, hi, lo, bin);
     ready = false;
+    if (n < 0) return kDrawRetry;
     if (tid == 0 && nrec < kDrawRecs) {
       D.rec_hi[nrec] = hi;
       D.rec_ct[nrec] = ct;
@@ -871,7 +868,8 @@ __device__ __forceinline__ uint32_t draw_ranked(DrawLds<NTH>& D, const SampleArg
       }
     }
     first = draw_block_min<NTH>(D, first);
-    const bool last = (k && seen + lim >= k) || lo <= kEnd || bin == (uint32_t)kDrawBins;
+    const bool last = (k && seen + lim >= k) || lo <= kDrawEnd || bin == (uint32_t)kDrawBins;
+    if (first == 0xffffffffu && last && !src.whole) return kDrawRetry;
     if (first != 0xffffffffu || last) {
       cnt = first != 0xffffffffu ? (int)first + 1 : lim;
       if (cnt == lim) {
@@ -895,7 +893,8 @@ __device__ __forceinline__ uint32_t draw_ranked(DrawLds<NTH>& D, const SampleArg
     hi = lo;
     __syncthreads();
   }
-  if (seen + cnt <= 0 || !(ct > 0.f) || !finitef_(ct)) return 0xffffffffu;
+  if (ct_out && tid == 0) *ct_out = ct;
+  if (seen + cnt <= 0 || !(ct > 0.f) || !finitef_(ct)) return kDrawFallback;
   const float target = clamp_uniform(cfg.u) * ct;
   // the inverse CDF: in the piece in LDS, or an earlier one gathered again
   if (target < ct0) {
@@ -911,13 +910,13 @@ __device__ __forceinline__ uint32_t draw_ranked(DrawLds<NTH>& D, const SampleArg
       if (q + 1 < nrec) {
         lo = D.rec_hi[q + 1];
       } else {
-        draw_descend<NTH>(D, r, hi);
+        if (!src.descend(D, hi)) return kDrawRetry;
         lo = D.lo;
       }
-      draw_gather<NTH>(D, r, lo, hi);
+      src.gather(D, lo, hi);
       n = draw_sort<NTH>(D, lo, hi);
       draw_folds<NTH>(D, n, n, 1.f, 0.f, c0);
-      if (target < D.end[1] || lo <= kEnd) break;
+      if (target < D.end[1] || lo <= kDrawEnd) break;
       c0 = D.end[1];
       hi = lo;
       ++q;
@@ -943,9 +942,65 @@ __device__ __forceinline__ uint32_t draw_ranked(DrawLds<NTH>& D, const SampleArg
     if (wf[(i / J) * ld + i % J] == w) same = min(same, (uint32_t)i);
   same = draw_block_min<NTH>(D, same);
   __syncthreads();
-  const uint32_t tok = draw_index<NTH>(D, r, w, pick - same, lo, hi);
+  const uint32_t tok = src.index(D, w, pick - same, lo, hi);
   __syncthreads();
   return tok;
+}
+
+// The whole draw (gpu.rs:820-899) for a top-p row, or a top-k row of more
+// than kBuf ranks.  Returns the token, or kDrawFallback for the argmax
+// fallback.  All threads call it.
+template <int NTH>
+__device__ __forceinline__ uint32_t draw_ranked(DrawLds<NTH>& D, const SampleArgs& a, int row, const RowCfg& cfg,
+                                                float M) {
+  const int tid = threadIdx.x;
+  const DrawRow r = draw_row<NTH>(a, row);
+  const DrawRowSrc<NTH> src{r, true};
+  const int span = 64 * kDrawPer * r.mult;
+  const int nt = (r.V + span - 1) / span;
+  draw_weights<NTH>(D, r, M, cfg.min_p);
+  const int k = cfg.cls == kTopK ? cfg.k_eff : 0;
+  const bool cut = cfg.cutoff < 1.f;
+  uint64_t lo = 0ull;
+  uint32_t bin;
+  bool ready = false;  // the first piece is gathered
+  float total;
+  if (k == 0) {
+    // the first piece: the bins of the nucleus by their mass (within 0.8%)
+    if (tid >= 64 && tid < 128) draw_predict<NTH>(D, nt);
+    if (tid < 64) {
+      float s = 0.f;
+      for (int t = tid; t < nt; t += 64) s += D.tsum[t];
+      draw_bins<NTH>(D, 0u, cut ? (cfg.cutoff * 1.008f + 0.002f) * wave_sum_f32(s) : __builtin_inff());
+    }
+    if (tid == 0) D.n = 0u;
+    __syncthreads();
+    bin = D.bnext;
+    lo = D.lo;
+    ready = bin != 0xffffffffu;
+    // (no first piece by the histogram: gather nothing)
+    draw_total<NTH>(D, r, ready ? lo : kDrawAll, kDrawAll);
+    total = D.total;
+  } else {
+    // the normaliser of the top k, in rank order
+    float t = -0.0f;
+    int seen = 0;
+    uint64_t hi = kDrawAll;
+    bin = 0u;
+    while (true) {
+      const int n = draw_piece<NTH>(D, src, hi, lo, bin);
+      draw_folds<NTH>(D, n, min(n, k - seen), 1.f, 0.f, t);
+      t = D.end[1];
+      seen += n;
+      if (seen >= k || lo <= kDrawEnd || bin == (uint32_t)kDrawBins) break;
+      hi = lo;
+    }
+    if (bin != 0xffffffffu) bin = 0u;  // from the top again
+    total = t;
+  }
+  __syncthreads();
+  if (!(total > 0.f) || !finitef_(total)) return kDrawFallback;
+  return draw_ranks<NTH>(D, src, cfg, k, total, ready, lo, bin, nullptr);
 }
 
 // The sum of the row's reference chunk [start, end): left to right from
@@ -1017,31 +1072,19 @@ __device__ __forceinline__ uint32_t draw_chunk_find(__amdgpu_buffer_rsrc_t s, in
   return chosen;
 }
 
-// Temperature-only rows: kernels.cu:7803-7867 with the exact weight
-// function: 256 contiguous chunks, a lane (or a quad) each, their serial
-// prefix, then the owning chunk again.  Returns the token or argmax_fin.
-// All threads call it.
+// The draw of a temperature-only row from its reference chunks' sums
+// (D.u.to.csum; the exponential's table in D.exptab): their serial prefix,
+// then the owning chunk again (kernels.cu:7834-7867).  Returns the token or
+// argmax_fin.  All threads call it.
 template <int NTH>
-__device__ __forceinline__ uint32_t draw_temperature(DrawLds<NTH>& D, const SampleArgs& a, int row, float M, float u,
-                                                     uint32_t argmax_fin) {
-  constexpr int Q = NTH / 256;
-  static_assert(Q == 1 || Q == 4, "a lane or a quad per reference chunk");
+__device__ __forceinline__ uint32_t draw_chunk_pick(DrawLds<NTH>& D, const DrawRow& r, float M, float u,
+                                                    uint32_t argmax_fin) {
   const int tid = threadIdx.x, lane = tid & 63;
-  const DrawRow r = draw_row<NTH>(a, row);
   const int V = r.V;
   const int chunk = (V + 255) / 256;
   float* csum = D.u.to.csum;
   float* prefix = D.u.to.prefix;
-  if (tid < 32) D.exptab[tid] = exp2_tab32((uint32_t)tid);
-  __syncthreads();
   const Exp2TabLds et{D.exptab};
-  {
-    const int t = tid / Q;
-    const int start = t * chunk, end = min(start + chunk, V);
-    const float s = draw_chunk_sum<Q>(r.s, start, end, M, et);
-    if ((tid & (Q - 1)) == 0) csum[t] = s;
-  }
-  __syncthreads();
   if (tid < 64) {
     float acc = 0.f;
     #pragma unroll 1
@@ -1079,6 +1122,32 @@ __device__ __forceinline__ uint32_t draw_temperature(DrawLds<NTH>& D, const Samp
   const uint32_t tok = D.token;
   __syncthreads();
   return tok != 0xffffffffu ? tok : argmax_fin;
+}
+
+// Temperature-only rows: kernels.cu:7803-7867 with the exact weight
+// function: 256 contiguous chunks, a lane (or a quad) each, then
+// draw_chunk_pick.  All threads call it.
+template <int NTH>
+__device__ __forceinline__ uint32_t draw_temperature(DrawLds<NTH>& D, const SampleArgs& a, int row, float M, float u,
+                                                     uint32_t argmax_fin) {
+  constexpr int Q = NTH / 256;
+  static_assert(Q == 1 || Q == 4, "a lane or a quad per reference chunk");
+  const int tid = threadIdx.x, lane = tid & 63;
+  const DrawRow r = draw_row<NTH>(a, row);
+  const int V = r.V;
+  const int chunk = (V + 255) / 256;
+  float* csum = D.u.to.csum;
+  if (tid < 32) D.exptab[tid] = exp2_tab32((uint32_t)tid);
+  __syncthreads();
+  const Exp2TabLds et{D.exptab};
+  {
+    const int t = tid / Q;
+    const int start = t * chunk, end = min(start + chunk, V);
+    const float s = draw_chunk_sum<Q>(r.s, start, end, M, et);
+    if ((tid & (Q - 1)) == 0) csum[t] = s;
+  }
+  __syncthreads();
+  return draw_chunk_pick<NTH>(D, r, M, u, argmax_fin);
 }
 
 }  // namespace hi_rocm

@@ -92,32 +92,18 @@ struct WideStat {
 
 static_assert(sizeof(WideStat) == 136, "WideStat layout");
 
-// Per (row, chunk) result of the wide pass for a top-p row: the maps of
-// the chunk's weights in the vocabulary-order fold for a start value in
-// binade e0, e0 + 1 or e0 + 2 (exact while the sum stays in that binade),
-// and the number of distinct-weight runs of the nucleus superset it wrote.
-constexpr int kCrossTerms = 48;  // terms of a crossing window
-constexpr int kCrossWins = 2;    // crossing windows a chunk records
+// Per (row, chunk) result of the wide pass for a top-p row: the number of
+// weights it listed (those of the nucleus superset) and, per tile of 1024
+// logits, its map in the vocabulary-order fold for a start in its predicted
+// binade, and in the one below (DrawLds in sampler_draw.h holds a row's).
+constexpr int kChunkTiles = 16;  // tiles of the largest chunk
 struct ChunkFold {
-  uint32_t e0;
-  uint32_t nruns;            // superset runs written; kFoldNone: the chunk's table overflowed
-  uint32_t has_end;          // chunk 0: `end` is the exact fold of its weights from -0.0
-  float end;
-  fold::Map map[3];          // the chunk's terms in binades e0, e0 + 1, e0 + 2
-  // the predicted crossings: nw windows (0: none predicted) around the
-  // terms where the fold leaves a binade; segment s (before window 0,
-  // between the windows, after the last) is folded in binade be[s] by its
-  // map seg[s]; window w holds wn[w] terms, added one by one
-  uint32_t nw;
-  uint32_t be[kCrossWins + 1];
-  uint32_t wn[kCrossWins];
-  fold::Map seg[kCrossWins + 1];
-  float term[kCrossWins][kCrossTerms];
-  uint32_t flags;            // bit k: map[k] holds the chunk's map; bit 3: the block maps are stored
-  uint32_t pad;
+  uint32_t n;
+  uint32_t pad[3];
+  fold::Map map[kChunkTiles], low[kChunkTiles];
+  uint32_t bin[kChunkTiles];
 };
-static_assert(sizeof(ChunkFold) == 480, "ChunkFold layout");
-constexpr uint32_t kFoldNone = 0xffffffffu;
+static_assert(sizeof(ChunkFold) == 336, "ChunkFold layout");
 
 struct SampleArgs {
   const void* logits;  // row 0 of the batch
@@ -144,12 +130,11 @@ struct SampleArgs {
   uint64_t* cand;      // [B][n_chunks][kFast]
   float* ws_s;         // [B][V]
   float* ws_w;         // [B][V]
-  uint64_t* ws_list;   // [B][list_stride]; the wide pass's superset runs
+  uint64_t* ws_list;   // [B][list_stride]; the wide pass's superset weights with their indexes
   int64_t list_stride;
   uint32_t* done;      // [kDoneRows] chunks of the row finished (zero between launches)
   WideStat* wstat;     // [B][n_chunks]
   ChunkFold* wfold;    // [B][n_chunks]
-  fold::Map* wbmap;    // [B][n_chunks][3][kScanThreads]: per-thread block maps of each ChunkFold binade
   uint32_t* diag;      // [B] how the wide pass finished each top-p row (WidePath)
   float* wtot;         // [B][2] the wide pass's normaliser and candidate total (debug export)
 };
@@ -159,11 +144,9 @@ struct SampleArgs {
 enum WidePath : uint32_t {
   kWideDone = 1,          // finished by the wide pass
   kWideNoStats = 2,       // a chunk's statistics were not written by this call's pass, or no finite logit
-  kWideChunkFull = 3,     // a chunk's table of distinct weights overflowed
   kWideTotal = 4,         // the normaliser is not positive and finite (argmax fallback)
-  kWideMergeFull = 5,     // the row's table of distinct weights overflowed
   kWideNoCutoff = 6,      // the cutoff lies outside the superset
-  kWideDrawFail = 7,      // the candidate total or the drawn index could not be resolved
+  kWideDrawFail = 7,      // the candidate total is not positive and finite
   // rows of the row kernel
   kRowPathMinp = 8,       // the min-p support finish
   kRowPathLists = 9,      // the candidate lists' finish (finish_core)
@@ -179,7 +162,7 @@ constexpr int kFusedMaxRows = kFusedMaxWorkgroups;
 constexpr int kDoneRows = 65536;
 
 struct WorkspaceLayout {
-  size_t stats, cand, ws_s, ws_w, ws_list, done, wstat, wfold, wbmap, diag, wtot, total;
+  size_t stats, cand, ws_s, ws_w, ws_list, done, wstat, wfold, diag, wtot, total;
   int64_t slots;       // (row, chunk) records reserved
   int64_t list_stride;
 };
@@ -205,7 +188,6 @@ inline WorkspaceLayout workspace_layout_slots(int max_batch, int V, int64_t slot
   L.stats = off; off = align(off + (size_t)L.slots * sizeof(ChunkStat));
   L.wstat = off; off = align(off + (size_t)L.slots * sizeof(WideStat));
   L.wfold = off; off = align(off + (size_t)L.slots * sizeof(ChunkFold));
-  L.wbmap = off; off = align(off + (size_t)L.slots * 3 * kScanThreads * sizeof(fold::Map));
   L.diag = off; off = align(off + (size_t)max_batch * sizeof(uint32_t));
   L.wtot = off; off = align(off + (size_t)max_batch * 2 * sizeof(float));
   L.cand = off; off = align(off + (size_t)L.slots * kFast * sizeof(uint64_t));
