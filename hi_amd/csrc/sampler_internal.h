@@ -110,7 +110,8 @@ struct SampleArgs {
   int dtype;
   int B, V;
   int64_t row_stride;  // elements between rows
-  int vec_ok;          // 128-bit (f32) / 64-bit (bf16) loads are aligned
+  int vec_ok;          // every row starts on 16 bytes (the general scan's wide loads)
+  int stream_ok;       // every element is aligned to its size (the select pass, the row kernel)
   ParamsView pv;
   const uint32_t* hoff;
   const uint32_t* hids;
@@ -167,7 +168,7 @@ struct WorkspaceLayout {
   int64_t list_stride;
 };
 
-int choose_chunk(int B, int V, int n_lp, int vec_ok, bool hist);
+int choose_chunk(int B, int V, int n_lp, int stream_ok, bool hist);
 
 inline int64_t next_pow2_i64(int64_t x) {
   int64_t p = 1;

@@ -951,7 +951,7 @@ size_t row_lds_bytes(int V) {
 
 bool row_kernel_fits(const SampleArgs& a) {
   return a.dtype == HI_ROCM_DTYPE_F32 && a.B >= kRowMinBatch && a.n_lp == 0 && a.out_token_lp == nullptr &&
-         a.vec_ok && a.chunk == kSelChunkLarge && a.V <= kRowMaxV && row_lds_bytes(a.V) <= kLdsPerCu;
+         a.stream_ok && a.chunk == kSelChunkLarge && a.V <= kRowMaxV && row_lds_bytes(a.V) <= kLdsPerCu;
 }
 
 template <bool MASK>

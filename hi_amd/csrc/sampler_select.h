@@ -318,6 +318,7 @@ __device__ __forceinline__ uint64_t wave_select(const Segs<NS>& sg, uint32_t nee
 typedef int i32x2_t __attribute__((ext_vector_type(2)));
 
 struct RowBuf {
+  int odd;  // 2: a bf16 row that starts between two words (its buffer starts 2 bytes earlier)
   __amdgpu_buffer_rsrc_t logits, mask;
 };
 
@@ -327,7 +328,13 @@ __device__ __forceinline__ RowBuf row_buf(const SampleArgs& a, int row, int c0, 
   RowBuf rb;
   const int esize = DT == HI_ROCM_DTYPE_BF16 ? 2 : 4;
   const char* base = (const char*)a.logits + ((int64_t)row * a.row_stride + c0) * esize;
-  rb.logits = __builtin_amdgcn_make_buffer_rsrc((void*)base, (short)0, (c1 - c0) * esize, kBufferConfig);
+  // the buffer starts on the word that holds the first logit and ends with
+  // the word that holds the last one; 16-byte loads need no more than that
+  // (the hardware checks each word's range by itself, so a load across the
+  // end returns the words before it)
+  rb.odd = (int)((uintptr_t)base & 2u);
+  rb.logits = __builtin_amdgcn_make_buffer_rsrc((void*)(base - rb.odd), (short)0, ((c1 - c0) * esize + rb.odd + 3) & ~3,
+                                                kBufferConfig);
   if (MASK)
     rb.mask = __builtin_amdgcn_make_buffer_rsrc((void*)(a.mask + (int64_t)row * a.mask_words + (c0 >> 5)),
                                                 (short)0, ((c1 - c0 + 31) >> 5) * 4, kBufferConfig);
@@ -993,7 +1000,7 @@ __device__ __forceinline__ void unpack16(const i32x4_t& r, float (&v)[EPL]) {
 template <int DT>
 __device__ __forceinline__ float load_one(const RowBuf& rb, uint32_t li) {
   if constexpr (DT == HI_ROCM_DTYPE_BF16)
-    return __uint_as_float((uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rb.logits, li * 2, 0, 0) << 16);
+    return __uint_as_float((uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rb.logits, (int)li * 2 + rb.odd, 0, 0) << 16);
   else
     return __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rb.logits, li * 4, 0, 0));
 }
@@ -1476,10 +1483,12 @@ __device__ __forceinline__ void select_chunk(const SampleArgs& a, int row, int c
   }
   const RowBuf rb = row_buf<DT, MASK>(a, row, c0, c0 + len);
   SelIn<NL> in;
+  uint32_t nx[NL] = {};  // bf16 rows that start between two words: the word after each load
   #pragma unroll
   for (int j = 0; j < NL; ++j) {
     const int li0 = (j * NT + tid) * EPL;
     in.raw[j] = __builtin_amdgcn_raw_buffer_load_b128(rb.logits, li0 * ESZ, 0, 0);
+    if (DT == HI_ROCM_DTYPE_BF16 && rb.odd) nx[j] = __builtin_amdgcn_raw_buffer_load_b32(rb.logits, li0 * ESZ + 16, 0, 0);
     if (MASK) in.mw[j] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rb.mask, (li0 >> 5) * 4, 0, 0);
   }
   const RowCfg cfg = load_cfg(a.pv, row, a.V, a.n_lp, a.need_lse);
@@ -1515,6 +1524,12 @@ __device__ __forceinline__ void select_chunk(const SampleArgs& a, int row, int c
   for (int j = 0; j < NL; ++j) {
     const int li0 = (j * NT + tid) * EPL;
     float v[EPL];
+    if (DT == HI_ROCM_DTYPE_BF16 && rb.odd) {
+      const uint32_t w0 = (uint32_t)in.raw[j][0], w1 = (uint32_t)in.raw[j][1], w2 = (uint32_t)in.raw[j][2],
+                     w3 = (uint32_t)in.raw[j][3];
+      in.raw[j] = i32x4_t{(int)__builtin_amdgcn_alignbit(w1, w0, 16u), (int)__builtin_amdgcn_alignbit(w2, w1, 16u),
+                          (int)__builtin_amdgcn_alignbit(w3, w2, 16u), (int)__builtin_amdgcn_alignbit(nx[j], w3, 16u)};
+    }
     unpack16<DT, EPL>(in.raw[j], v);
     if (MASK) {
       const uint32_t bits = in.mw[j] >> (li0 & 31);
