@@ -905,6 +905,153 @@ __device__ __noinline__ void row_general(KernargSampleArgs* ap, int row) {
   general_row_path<MASK>(a, row, lds_raw);
 }
 
+// Rows of other classes than top-k, by all of the workgroup's threads: one
+// pass over the logits (mask; the history's tokens out of band from a hash
+// of their counts) leaves the scaled logits in ws_s with their maximum and
+// argmax, then the greedy token or the draws of sampler_draw.h.  On the first
+// four waves, in 8192-logit chunks of the select pass (row_general), 256
+// rows of 151,936 took 133 us (greedy), 248 (temperature only), 505 (nucleus)
+// and 460 (min-p); here 61, 135, 260 and 237 us.  Bound: the exact
+// exponentials (about 33 us a row and CU) and the two later passes over the
+// weights.
+// Returns false for what row_general resolves: a history too long for the
+// hash, no finite scaled logit, the argmax fallback.
+constexpr int kRowHashBits = 12;
+constexpr int kRowHash = 1 << kRowHashBits;
+struct RowWideLds {
+  uint32_t hkey[kRowHash], hcnt[kRowHash];  // history ids (~0: free) and their summed counts
+  uint32_t bits[kRowMaxV / 32];             // history marks
+  uint32_t red[kRowWaves];
+  uint64_t red64[kRowWaves];
+};
+
+template <bool MASK>
+__device__ __noinline__ bool row_wide(KernargSampleArgs* ap, int row) {
+  extern __shared__ __align__(16) unsigned char lds_raw[];
+  SampleArgs a;
+  {
+    typedef const __attribute__((address_space(4))) uint64_t KernargWord;
+    KernargWord* w = (KernargWord*)ap;
+    uint64_t* d = reinterpret_cast<uint64_t*>(&a);
+    #pragma unroll
+    for (int i = 0; i < (int)(sizeof(SampleArgs) / 8); ++i) d[i] = w[i];
+  }
+  RowWideLds& L = *reinterpret_cast<RowWideLds*>(lds_raw);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int V = a.V;
+  const RowCfg cfg = load_cfg(a.pv, row, V, 0, 0);
+  const DrawRow r = draw_row<kRowThreads>(a, row);
+  const float* lrow = (const float*)a.logits + (int64_t)row * a.row_stride;
+  const __amdgpu_buffer_rsrc_t lg = __builtin_amdgcn_make_buffer_rsrc((void*)lrow, 0, V * 4, kBufferConfig);
+  const uint32_t* mrow = MASK ? a.mask + (int64_t)row * a.mask_words : nullptr;
+  uint32_t h0 = 0u, h1 = 0u;
+  if (a.hoff) { h0 = a.hoff[row]; h1 = a.hoff[row + 1]; }
+  const bool hist = h1 > h0;
+  if (h1 > h0 + (uint32_t)(kRowHash * 3 / 4)) return false;
+  if (hist) {
+    for (int i = tid; i < kRowHash; i += kRowThreads) { L.hkey[i] = 0xffffffffu; L.hcnt[i] = 0u; }
+    for (int i = tid; i < (V + 31) / 32; i += kRowThreads) L.bits[i] = 0u;
+    __syncthreads();
+    for (uint32_t h = h0 + (uint32_t)tid; h < h1; h += kRowThreads) {
+      const uint32_t id = a.hids[h];
+      if (id >= (uint32_t)V) continue;
+      atomicOr(&L.bits[id >> 5], 1u << (id & 31u));
+      uint32_t s = (id * 0x9E3779B1u) >> (32 - kRowHashBits);
+      while (true) {  // (at most 3/4 of the slots are ever taken)
+        const uint32_t old = atomicCAS(&L.hkey[s], 0xffffffffu, id);
+        if (old == 0xffffffffu || old == id) break;
+        s = (s + 1u) & (uint32_t)(kRowHash - 1);
+      }
+      atomicAdd(&L.hcnt[s], a.hcnt[h]);
+    }
+    __syncthreads();
+  }
+  const bool store = cfg.cls != kGreedy;
+  const bool fin = cfg.cls != kGreedy || a.pv.greedy_rule == kGreedyFiniteLane;  // which argmax
+  uint32_t kmax = 0u;  // the largest key of a finite logit
+  float bv = -__builtin_inff();
+  uint32_t bo = 0xffffffffu;  // the argmax's value, and its place among equals
+  // -0 and +0 compare equal; IEEE: the first maximum above -inf (NaN never);
+  // finite lanes: by their order
+  auto stat = [&](float v, int i, bool on, bool max_too) {
+    const bool f = finitef_(v);
+    if (max_too) kmax = max(kmax, f && on ? okey(v) : 0u);
+    const uint32_t o = fin ? fin_order((uint32_t)i) : (uint32_t)i;
+    const bool take = on && (fin ? f : v > -__builtin_inff()) && (v > bv || (v == bv && o < bo));
+    bv = take ? v : bv;
+    bo = take ? o : bo;
+  };
+  auto pass = [&](auto st) {
+    constexpr bool kStore = decltype(st)::value;
+    draw_stream<kRowThreads>(r, lg, [&](int, int, int c0, const float (&x)[4][4]) {
+      #pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = c0 + j * 256 + lane * 4;
+        uint32_t keep = 0xfu;
+        if (MASK) keep = i < V ? mrow[i >> 5] >> (i & 31) : 0u;
+        uint32_t mark = 0u;
+        if (hist) mark = i < V ? L.bits[i >> 5] >> (i & 31) : 0u;
+        i32x4_t o;
+        #pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float v = (keep >> q) & 1u ? x[j][q] : -__builtin_inff();
+          stat(v, i + q, !((mark >> q) & 1u) && i + q < V, kStore || MASK);
+          if (kStore) o[q] = __float_as_int(finitef_(v) ? v / cfg.t_eff : -__builtin_inff());
+        }
+        // (history tokens are stored again below; a lane's access that
+        // crosses the row's end stores nothing)
+        if (kStore) __builtin_amdgcn_raw_buffer_store_b128(o, r.s, i + 4 <= V ? i * 4 : 0x7ffffff0, 0, 0);
+      }
+    });
+  };
+  if (store) pass(std::true_type{});
+  else pass(std::false_type{});
+  if (store && tid < (V & 3)) {
+    const int i = (V & ~3) + tid;
+    const bool on = !MASK || ((mrow[i >> 5] >> (i & 31)) & 1u);
+    const float v = on ? lrow[i] : -__builtin_inff();
+    __builtin_amdgcn_raw_buffer_store_b32((uint32_t)__float_as_int(finitef_(v) ? v / cfg.t_eff : -__builtin_inff()), r.s, i * 4, 0, 0);
+  }
+  if (hist) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stream's stores are ordered before these
+    __syncthreads();
+    for (int s = tid; s < kRowHash; s += kRowThreads) {
+      const uint32_t id = L.hkey[s];
+      if (id == 0xffffffffu) continue;
+      const bool on = !MASK || ((mrow[id >> 5] >> (id & 31u)) & 1u);
+      const float v = apply_penalties(on ? lrow[id] : -__builtin_inff(), L.hcnt[s], cfg);
+      stat(v, (int)id, true, true);
+      if (store)
+        __builtin_amdgcn_raw_buffer_store_b32((uint32_t)__float_as_int(finitef_(v) ? v / cfg.t_eff : -__builtin_inff()), r.s, (int)id * 4, 0, 0);
+    }
+  }
+  kmax = block_max_u32<kRowThreads>(kmax, L.red);
+  const uint64_t best = block_max_u64<kRowThreads>(
+      bo == 0xffffffffu ? 0ull : ((uint64_t)okey(bv == 0.f ? 0.f : bv) << 32) | (uint64_t)(0xffffffffu - bo), L.red64);
+  const uint32_t order = 0xffffffffu - (uint32_t)best;
+  const uint32_t am = best == 0ull ? 0u : (fin ? fin_index(order) : order);
+  uint32_t token;
+  if (MASK && kmax == 0u) {
+    token = cfg.eos;
+  } else if (cfg.cls == kGreedy) {
+    token = am;
+  } else {
+    const float M = kmax == 0u ? -__builtin_inff() : okey_inv(kmax) / cfg.t_eff;
+    if (!finitef_(M)) return false;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    DrawLds<kRowThreads>& D = *reinterpret_cast<DrawLds<kRowThreads>*>(lds_raw);
+    token = cfg.cls == kTempOnly ? draw_temperature<kRowThreads>(D, a, row, M, cfg.u, am)
+                                 : draw_ranked<kRowThreads>(D, a, row, cfg, M);
+    if (token == kDrawFallback) return false;
+  }
+  if (tid == 0) {
+    a.out_tokens[row] = token;
+    a.diag[row] = kRowPathGeneral;
+  }
+  return true;
+}
+
 // The row kernel's arguments as its argument segment lays them out: each at
 // the next offset aligned for its type, as in this struct.
 struct RowKernelArgs {
@@ -935,16 +1082,23 @@ __global__ void __launch_bounds__(kRowThreads) row_kernel(const void* logits, in
     if (row_stream<MASK>(L, a, row, cfg, lds_raw, pp)) return;
     __syncthreads();
   }
-  if (threadIdx.x >= NT) return;
   typedef const __attribute__((address_space(4))) char KernargByte;
-  row_general<MASK>(
-      (KernargSampleArgs*)((KernargByte*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(RowKernelArgs, a)), row);
+  KernargSampleArgs* ka =
+      (KernargSampleArgs*)((KernargByte*)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(RowKernelArgs, a));
+  if (cfg.cls != kTopK) {
+    if (row_wide<MASK>(ka, row)) return;
+    __syncthreads();
+  }
+  if (threadIdx.x >= NT) return;
+  row_general<MASK>(ka, row);
 }
 
 size_t row_lds_bytes(int V) {
   const size_t fast = kRowHead + sizeof(uint2) * ((V + 31) / 32);
   const size_t general = kSelHead + sel_hist_bytes(kSelChunkLarge);
   size_t b = fast > general ? fast : general;
+  b = b > sizeof(RowWideLds) ? b : sizeof(RowWideLds);
+  b = b > sizeof(DrawLds<kRowThreads>) ? b : sizeof(DrawLds<kRowThreads>);
   return b > sizeof(FinLds) ? b : sizeof(FinLds);
 }
 

@@ -63,3 +63,49 @@ def test_draw_parity(hip, oracle, V, kind):
         got = out["tokens"].cpu().numpy().view(np.uint32)
         bad = np.flatnonzero(got != want)
         assert bad.size == 0, (bad, got[bad], want[bad])
+
+
+@pytest.mark.parametrize("with_mask", [False, True])
+def test_row_kernel_other_classes(hip, oracle, with_mask):
+    """256 rows of an odd vocabulary in one workgroup each: every class but
+    the streamed top-k, with histories (repeated ids, ids past the
+    vocabulary, one longer than the kernel's table), penalties, masks (one
+    row fully masked), rows without a finite logit, infinities and NaN."""
+    import torch
+    from hi_amd import sampler as S
+    B, V = 256, 65537
+    rng = np.random.default_rng(9 + with_mask)
+    x = _rows("spiked", B, V, 5)
+    p = _params(B)
+    p["temperature"][0::7] = 0.0
+    p["eos_id"] = 3
+    p["repetition_penalty"][1::3] = 1.2
+    p["frequency_penalty"][1::2] = 0.1
+    x[3, :] = -np.inf
+    x[8, 17] = np.inf
+    x[13, 5] = np.nan
+    x[14, :] = np.round(x[14, :])
+    off, ids, cnt = [0], [], []
+    for b in range(B):
+        n = 3500 if b == 20 else (0 if b % 4 == 0 else int(rng.integers(1, 300)))
+        i = rng.integers(0, V + 50, n)
+        if n:
+            i[:8] = np.argsort(np.nan_to_num(x[b], nan=-1e30, posinf=-1e30))[-8:][:n]  # likely tokens penalised
+        ids.append(np.concatenate([i, i[:5]]).astype(np.uint32))
+        cnt.append(rng.integers(1, 4, len(ids[-1])).astype(np.uint32))
+        off.append(off[-1] + len(ids[-1]))
+    off, ids, cnt = np.array(off, np.uint32), np.concatenate(ids), np.concatenate(cnt)
+    mask = None
+    if with_mask:
+        mask = rng.integers(0, 2 ** 32, (B, (V + 31) // 32), dtype=np.uint64).astype(np.uint32)
+        mask[30] = 0
+    u = rng.random(B).astype(F32)
+    i32 = lambda a: torch.from_numpy(a.view(np.int32)).cuda()  # noqa: E731
+    print(f"row kernel classes mask={with_mask}", flush=True)
+    out = S.Sampler(B, V).sample(torch.from_numpy(x).cuda(), S.params_to_device(p), torch.from_numpy(u).cuda(),
+                                 i32(off), i32(ids), i32(cnt), None if mask is None else i32(mask))
+    torch.cuda.synchronize()
+    want = oracle.sample_rows(x, p, u, off, ids, cnt, mask)["tokens"]
+    got = out["tokens"].cpu().numpy().view(np.uint32)
+    bad = np.flatnonzero(got != want)
+    assert bad.size == 0, (bad, got[bad], want[bad])
