@@ -51,3 +51,58 @@ def test_spec_verify_parity(hip, oracle, B, K, V):
         for b in range(B):
             assert np.array_equal(tt[b, :cc[b]], wt[b, :wc[b]]), b
             assert (tt[b, cc[b]:] == 0xffffffff).all(), "write past the emitted tokens"
+
+
+@pytest.mark.parametrize("V", [1, 8191, 8193, 50257, 70001])
+def test_spec_verify_parts(hip, oracle, V):
+    """Rows split over workgroups (8192 logits each) and, inside a capture
+    whose stream has no buffer yet, one workgroup a row: maxima on both
+    sides of every part's edge, equal maxima in two parts, -inf and NaN
+    rows; the capture replayed three times."""
+    import torch
+    lib = hip.load()
+    B, K = 6, 2
+    rng = np.random.default_rng(V)
+    x = (rng.standard_normal((B, K + 1, V)) * 2).astype(F32)
+    edges = [i for i in (0, 8191, 8192, V - 1) if i < V]
+    for n, e in enumerate(edges):
+        x[n % B, n % (K + 1), e] = 50.0
+    x[4, 0, edges] = 60.0
+    x[5, 0, :] = -np.inf
+    x[5, 1, :] = np.nan
+    x[5, 2, V // 2:] = np.nan
+    d = rng.integers(0, V, (B, K)).astype(np.uint32)
+    wg, wt, wc = oracle.spec_verify_greedy(x, d, None)
+    d[:, 0] = wg[:, 0]
+    wg, wt, wc = oracle.spec_verify_greedy(x, d, None)
+    dx, dd = torch.from_numpy(x).cuda(), torch.from_numpy(d.view(np.int32)).cuda()
+    g, t = (torch.full((B, K + 1), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+    c = torch.full((B,), -1, dtype=torch.int32, device="cuda")
+
+    def call(s):
+        hip.check(lib.hi_rocm_spec_verify_greedy(dx.data_ptr(), B, K, V, dd.data_ptr(), 0, g.data_ptr(), t.data_ptr(),
+                                                 c.data_ptr(), s.cuda_stream))
+
+    def same():
+        assert np.array_equal(g.cpu().numpy().view(np.uint32), wg)
+        assert np.array_equal(c.cpu().numpy(), wc)
+        tt = t.cpu().numpy().view(np.uint32)
+        assert all(np.array_equal(tt[b, :wc[b]], wt[b, :wc[b]]) for b in range(B))
+
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    print(f"spec verify parts V={V}", flush=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        call(s)
+    for _ in range(3):
+        g.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        same()
+    for _ in range(2):
+        g.fill_(-1)
+        torch.cuda.synchronize()
+        call(s)
+        s.synchronize()
+        same()
