@@ -3,6 +3,8 @@ restatement of gpu.rs:10725-10762 (host argmax gpu.rs:6406-6435): per-row
 argmax, accepted counts and emitted tokens bit for bit, over drafts that
 are fully accepted, rejected at each position, per-request draft lengths,
 K = 0, ties, NaN and infinities, and a 151,936-token vocabulary."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -89,7 +91,9 @@ def test_spec_verify_parts(hip, oracle, V):
         tt = t.cpu().numpy().view(np.uint32)
         assert all(np.array_equal(tt[b, :wc[b]], wt[b, :wc[b]]) for b in range(B))
 
-    s = torch.cuda.Stream()
+    handle = ctypes.c_uint64()  # a stream of its own: torch's come from a pool and may already hold a buffer
+    assert int(torch.cuda.cudart().cudaStreamCreate(ctypes.addressof(handle))) == 0
+    s = torch.cuda.ExternalStream(handle.value)
     torch.cuda.synchronize()
     print(f"spec verify parts V={V}", flush=True)
     graph = torch.cuda.CUDAGraph()
@@ -106,3 +110,6 @@ def test_spec_verify_parts(hip, oracle, V):
         call(s)
         s.synchronize()
         same()
+    hip.check(lib.hi_rocm_sampler_release(s.cuda_stream))
+    del graph, s
+    assert int(torch.cuda.cudart().cudaStreamDestroy(handle.value)) == 0
