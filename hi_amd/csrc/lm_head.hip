@@ -44,6 +44,7 @@ static_assert(sizeof(LmTileRec) == 32, "LmTileRec layout");
 // Loads of one K block for a lane: 16 bytes at element `off` of each operand
 // row (rows past the batch or the vocabulary read row 0 and are dropped in
 // the epilogue, so every load is unconditional).
+// (Weights by nontemporal loads, though read once: one row 222 -> 237 us.)
 __device__ __forceinline__ lm_bf16x8 lm_ld(const __bf16* p) { return *reinterpret_cast<const lm_bf16x8*>(p); }
 
 // The logits of vocabulary columns [tile0, tile0 + kLmTile) for rows
@@ -72,7 +73,12 @@ __device__ __forceinline__ lm_bf16x8 lm_ld(const __bf16* p) { return *reinterpre
 template <int RG>
 __device__ __forceinline__ void lm_gemm_tile(const LmArgs& a, int tile0, float* tile) {
   static_assert(kLmThreads == 128, "hidden block staging: 128 threads x 32 bytes per row group");
-  __shared__ __align__(16) __bf16 a_lds[2][RG * 32 * 64];
+  // the ring lies in the tile's own LDS, which is written after the last
+  // product: 32 KB a workgroup instead of 48 at RG = 2, so four instead of
+  // three share a CU (64 rows, H = 4096, V = 151,936, fused: 350 -> 330 us;
+  // three waves a SIMD would spill: 872)
+  __bf16 (*a_lds)[RG * 32 * 64] = reinterpret_cast<__bf16 (*)[RG * 32 * 64]>(tile);
+  static_assert(2 * RG * 32 * 64 * sizeof(__bf16) <= RG * 32 * kLmTile * sizeof(float), "the ring fits the tile");
   const int tid = threadIdx.x;
   const int lane = tid & 63, wid = tid >> 6;
   const int r = lane & 15, g = lane >> 4;
@@ -182,6 +188,7 @@ __device__ __forceinline__ void lm_gemm_tile(const LmArgs& a, int tile0, float* 
           acc[q][mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(at[mt], bt[nt], acc[q][mt][nt], 0, 0, 0);
     }
   }
+  __syncthreads();  // both waves have read the ring's last block
   // epilogue: bias, softcap; tile[m * kLmTile + column]
   #pragma unroll
   for (int q = 0; q < RG; ++q)
