@@ -183,6 +183,11 @@ void carve(hi_rocm::SampleArgs& a, void* ws, const hi_rocm::WorkspaceLayout& L) 
   a.wfold = (hi_rocm::ChunkFold*)(base + L.wfold);
   a.diag = (uint32_t*)(base + L.diag);
   a.wtot = (float*)(base + L.wtot);
+  // Masked rows that do not start on 16 bytes stay with the general scan: the
+  // streaming passes send rows of few allowed tokens to their exact fallback
+  // (12 f32 top-k rows of 100,003: 56 us scanned, 134 streamed; 250 rows of
+  // 64,001: 120 and 250).
+  if (a.mask != nullptr && !a.vec_ok) a.stream_ok = 0;
   a.chunk = hi_rocm::choose_chunk(a.B, a.V, a.n_lp, a.stream_ok, a.hoff != nullptr);
   a.n_chunks = (a.V + a.chunk - 1) / a.chunk;
 }
@@ -190,7 +195,7 @@ void carve(hi_rocm::SampleArgs& a, void* ws, const hi_rocm::WorkspaceLayout& L) 
 // Rows that start on 16 bytes take the general scan's wide loads.  The
 // streaming passes read 16 bytes from any 4-byte aligned place (and bf16 rows
 // that start between two words shift them), so they take every row whose
-// elements are aligned: an odd vocabulary's rows ran the general scan and a
+// elements are aligned (masked ones: carve): an odd vocabulary's rows ran the general scan and a
 // one-workgroup finish before (64 top-k rows of 50,257: 37 -> 20 us, top-k 1024 236 -> 51 us).
 int vec_aligned(const void* p, int dtype, int64_t row_stride) {
   const int64_t esize = dtype == HI_ROCM_DTYPE_BF16 ? 2 : 4;

@@ -65,15 +65,16 @@ def test_draw_parity(hip, oracle, V, kind):
         assert bad.size == 0, (bad, got[bad], want[bad])
 
 
-@pytest.mark.parametrize("with_mask", [False, True])
-def test_row_kernel_other_classes(hip, oracle, with_mask):
-    """256 rows of an odd vocabulary in one workgroup each: every class but
+@pytest.mark.parametrize("with_mask,V", [(False, 65537), (True, 65540), (True, 65537)])
+def test_row_kernel_other_classes(hip, oracle, with_mask, V):
+    """256 rows in one workgroup each (masked rows of an odd vocabulary: the
+    general scan): every class but
     the streamed top-k, with histories (repeated ids, ids past the
     vocabulary, one longer than the kernel's table), penalties, masks (one
     row fully masked), rows without a finite logit, infinities and NaN."""
     import torch
     from hi_amd import sampler as S
-    B, V = 256, 65537
+    B = 256
     rng = np.random.default_rng(9 + with_mask)
     x = _rows("spiked", B, V, 5)
     p = _params(B)
