@@ -111,7 +111,7 @@ struct SampleArgs {
   int B, V;
   int64_t row_stride;  // elements between rows
   int vec_ok;          // every row starts on 16 bytes (the general scan's wide loads)
-  int stream_ok;       // every element is aligned to its size (the select pass, the row kernel)
+  int stream_ok;       // every element is aligned to its size, and masked rows start on 16 bytes (the select pass, the row kernel)
   ParamsView pv;
   const uint32_t* hoff;
   const uint32_t* hids;
