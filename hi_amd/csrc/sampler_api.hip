@@ -70,15 +70,17 @@ hipError_t zero_counters(void* ws, int n, hipStream_t stream) {
 struct DeviceWorkspace {
   void* ptr = nullptr;
   size_t bytes = 0;
-  // buffers outgrown but kept until release (kWsVerify: a captured graph may
-  // hold them; each is at least twice the one before)
-  std::vector<void*> old;
 };
-using hi_rocm::kWsIndexer;
-using hi_rocm::kWsSampler;
+// Buffers of a (device, stream): the sampler's, and the DSV4 indexer's
+// (a few KB per 4096 scores; its histogram kept at zero between calls).
+enum WsKind { kWsSampler = 0, kWsIndexer = 1 };
 std::mutex g_ws_mutex;
 std::map<std::tuple<int, uintptr_t, int>, DeviceWorkspace> g_ws;
 
+// The stream's buffer of `kind`, at least `bytes`, with its first
+// zero_words words zero after a growth.  When it would grow during capture:
+// an error, or with `optional` success and *out = nullptr (the caller takes
+// a path without it).
 int stream_buffer(int kind, size_t bytes, int zero_words, bool optional, hipStream_t stream, void** out) {
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
@@ -98,12 +100,6 @@ int stream_buffer(int kind, size_t bytes, int zero_words, bool optional, hipStre
                   "hi-rocm: the stream's sampler workspace would grow to " + std::to_string(bytes) +
                       " bytes during stream capture (an allocation); call hi_rocm_sampler_reserve with the "
                       "largest shape before capturing");
-    if (kind == hi_rocm::kWsVerify) {
-      bytes = std::max({bytes, 2 * ws.bytes, (size_t)1 << 20});
-      if (ws.ptr) ws.old.push_back(ws.ptr);
-      ws.ptr = nullptr;
-      ws.bytes = 0;
-    }
     if (ws.ptr) {
       e = hipStreamSynchronize(stream);
       if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
@@ -114,7 +110,7 @@ int stream_buffer(int kind, size_t bytes, int zero_words, bool optional, hipStre
     }
     e = hipMalloc(&ws.ptr, bytes);
     if (e != hipSuccess) return hip_fail(e, "hipMalloc(sampler workspace)");
-    if (zero_words > 0) e = zero_counters(ws.ptr, zero_words, stream);
+    e = zero_counters(ws.ptr, zero_words, stream);
     if (e != hipSuccess) return hip_fail(e, "sampler workspace counter reset");
     ws.bytes = bytes;
   }
@@ -132,12 +128,9 @@ int release_workspace(hipStream_t stream) {
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
   std::lock_guard<std::mutex> lock(g_ws_mutex);
-  std::vector<decltype(g_ws)::iterator> held;
-  for (int k = 0; k < hi_rocm::kWsKinds; ++k) {
-    const auto it = g_ws.find(std::make_tuple(dev, (uintptr_t)stream, k));
-    if (it != g_ws.end()) held.push_back(it);
-  }
-  if (held.empty()) return HI_ROCM_OK;
+  auto it0 = g_ws.find(std::make_tuple(dev, (uintptr_t)stream, (int)kWsSampler));
+  auto it1 = g_ws.find(std::make_tuple(dev, (uintptr_t)stream, (int)kWsIndexer));
+  if (it0 == g_ws.end() && it1 == g_ws.end()) return HI_ROCM_OK;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   e = hipStreamIsCapturing(stream, &cs);
   if (e != hipSuccess) return hip_fail(e, "hipStreamIsCapturing");
@@ -145,12 +138,8 @@ int release_workspace(hipStream_t stream) {
     return fail(HI_ROCM_ERR_UNSUPPORTED, "hi_rocm_sampler_release: the stream is being captured");
   e = hipStreamSynchronize(stream);
   if (e != hipSuccess) return hip_fail(e, "hipStreamSynchronize");
-  for (auto it : held) {
-    for (void* p : it->second.old) {
-      e = hipFree(p);
-      if (e != hipSuccess) return hip_fail(e, "hipFree");
-    }
-    it->second.old.clear();
+  for (auto it : {it0, it1}) {
+    if (it == g_ws.end()) continue;
     if (it->second.ptr) {
       e = hipFree(it->second.ptr);
       if (e != hipSuccess) return hip_fail(e, "hipFree");
@@ -159,16 +148,6 @@ int release_workspace(hipStream_t stream) {
   }
   return HI_ROCM_OK;
 }
-
-}  // namespace
-
-namespace hi_rocm {
-int api_stream_buffer(int kind, size_t bytes, int zero_words, bool optional, hipStream_t stream, void** out) {
-  return stream_buffer(kind, bytes, zero_words, optional, stream, out);
-}
-}  // namespace hi_rocm
-
-namespace {
 
 void carve(hi_rocm::SampleArgs& a, void* ws, const hi_rocm::WorkspaceLayout& L) {
   char* base = (char*)ws;

@@ -244,16 +244,6 @@ hipError_t launch_debug_distribution(const SampleArgs& a, float* out_proc, float
 int api_fail(int code, const char* msg);
 int api_hip_fail(hipError_t e, const char* where);
 
-// Buffers the library keeps per (device, stream): the sampler's workspace of
-// the mirrors, the DSV4 indexer's (its histogram kept at zero between
-// calls), and the draft verification's parts.
-enum WsKind { kWsSampler = 0, kWsIndexer = 1, kWsVerify = 2, kWsKinds = 3 };
-// The stream's buffer of `kind`, at least `bytes`, with its first zero_words
-// words zero after a growth.  When it would grow during capture: an error, or
-// with `optional` success and *out = nullptr (the caller takes a path without
-// it).
-int api_stream_buffer(int kind, size_t bytes, int zero_words, bool optional, hipStream_t stream, void** out);
-
 // The LM-head projection + bias + softcap fused into the sampler's first
 // pass (sampler_kernels.hip).
 constexpr int kLmTile = 128;     // vocabulary columns per workgroup (chunk)

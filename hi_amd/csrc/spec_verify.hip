@@ -10,13 +10,15 @@
 // accepts draft[i] while it equals greedy[i], and emits
 // greedy[0 ..= accepted] (the first mismatch's target token, or the bonus
 // token after a fully accepted draft).  Here the rows are split over
-// workgroups (one workgroup a row left most of the chip idle), and one
-// workgroup per request then merges its rows' parts and runs the acceptance,
-// so only the emitted tokens and their count leave the device.
+// workgroups (one workgroup a row left most of the chip idle), which merge
+// their maxima in the caller's out_greedy, and one workgroup per request then
+// runs the acceptance.  Calls with different outputs share nothing, whatever
+// streams, threads or graphs they run on, and only the emitted tokens and
+// their count leave the device.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <mutex>
+#include <algorithm>
 
 #include "hi_rocm.h"
 #include "sampler_internal.h"
@@ -24,8 +26,6 @@
 
 namespace hi_rocm {
 namespace {
-
-constexpr int kVerifyThreads = 256;
 
 // Order key of a non-NaN float with -0 taken as +0 (the reference's '>'
 // does not tell them apart).
@@ -40,6 +40,10 @@ __device__ __forceinline__ uint32_t order_key0(float x) {
 __device__ __forceinline__ uint64_t verify_key(float v, uint32_t i) {
   return ((uint64_t)order_key0(v) << 32) | (uint64_t)(0xffffffffu - i);
 }
+__device__ __forceinline__ float verify_value(uint64_t key) {
+  const uint32_t o = (uint32_t)(key >> 32);
+  return __uint_as_float((o & 0x80000000u) ? o ^ 0x80000000u : ~o);
+}
 __device__ __forceinline__ uint64_t verify_wave_max(uint64_t best) {
   #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
@@ -52,25 +56,28 @@ __device__ __forceinline__ uint64_t verify_wave_max(uint64_t best) {
 }
 
 // The key of the row's first maximum above -inf in [i0, i1) (0: none), by a
-// workgroup of kVerifyThreads: range-checked 16-byte loads, kVerifyLoads a
-// thread in flight.
+// workgroup of T threads: range-checked 16-byte loads, kVerifyLoads a thread
+// in flight.  ahead() is called behind the first ones.
 constexpr int kVerifyLoads = 8;
-constexpr int kVerifySpan = kVerifyThreads * 4 * kVerifyLoads;  // logits of a step
-__device__ __forceinline__ uint64_t verify_span_max(const float* x, int V, int i0, int i1, uint64_t* red) {
+template <int T>
+constexpr int kVerifySpan = T * 4 * kVerifyLoads;  // logits of a step
+template <int T, typename AheadF>
+__device__ __forceinline__ uint64_t verify_span_max(const float* x, int V, int i0, int i1, uint64_t* red, AheadF ahead) {
   const int tid = threadIdx.x;
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, V * 4, kBufferConfig);
   float bv = -__builtin_inff();
   uint32_t bi = 0xffffffffu;
-  for (int b = i0; b < i1; b += kVerifySpan) {
+  for (int b = i0; b < i1; b += kVerifySpan<T>) {
     i32x4_t v[kVerifyLoads];
     #pragma unroll
     for (int j = 0; j < kVerifyLoads; ++j)
-      v[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, (b + (j * kVerifyThreads + tid) * 4) * 4, 0, 0);
+      v[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, (b + (j * T + tid) * 4) * 4, 0, 0);
+    if (b == i0) ahead();
     #pragma unroll
     for (int j = 0; j < kVerifyLoads; ++j) {
       #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int i = b + (j * kVerifyThreads + tid) * 4 + q;
+        const int i = b + (j * T + tid) * 4 + q;
         const float f = __int_as_float(v[j][q]);
         const bool take = f > bv && i < V;  // (NaN never; a thread's indices rise)
         bv = take ? f : bv;
@@ -83,68 +90,95 @@ __device__ __forceinline__ uint64_t verify_span_max(const float* x, int V, int i
   __syncthreads();
   best = red[0];
   #pragma unroll
-  for (int w = 1; w < kVerifyThreads / 64; ++w) best = red[w] > best ? red[w] : best;
+  for (int w = 1; w < T / 64; ++w) best = red[w] > best ? red[w] : best;
   return best;
 }
 
-// The row's answer from its key: index 0 with a NaN there, or when nothing
-// is above -inf.
-__device__ __forceinline__ uint32_t verify_index(uint64_t best, float x0) {
-  return x0 != x0 || best == 0ull ? 0u : 0xffffffffu - (uint32_t)best;
+// Makes key's index the row's answer unless the answer comes before it (the
+// larger value, then the lower index).  Whatever the caller's array holds at
+// the start is no more than one more index to compare with: one of the row's
+// stands for its own logit, any other (or a NaN's) gives way.  An index once
+// taken only gives way to an earlier one, so the loop ends after at most one
+// round per other part, and the result does not depend on their order.
+// `cur`: the answer seen last.
+__device__ __forceinline__ void verify_take(const float* x, int V, uint64_t key, uint32_t cur, float xc,
+                                            uint32_t* answer) {
+  const float bv = verify_value(key);
+  const uint32_t bi = 0xffffffffu - (uint32_t)key;
+  while (true) {
+    if (xc > bv || (xc == bv && cur <= bi)) return;
+    if (__hip_atomic_compare_exchange_strong(answer, &cur, bi, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT))
+      return;
+    xc = cur < (uint32_t)V ? x[cur] : -__builtin_inff();
+  }
 }
 
-// The key of part `blockIdx.x` (of `span` logits) of verify row blockIdx.y.
-__global__ void __launch_bounds__(kVerifyThreads)
-    verify_part_kernel(const float* logits, int V, int span, uint64_t* parts) {
-  __shared__ uint64_t red[kVerifyThreads / 64];
-  const int64_t r = blockIdx.y;
-  const int i0 = (int)blockIdx.x * span;
-  const uint64_t best = verify_span_max(logits + r * V, V, i0, min(i0 + span, V), red);
-  if (threadIdx.x == 0) parts[r * gridDim.x + blockIdx.x] = best;
+// Part blockIdx.x % n_parts (of `span` logits) of verify row blockIdx.x /
+// n_parts.
+template <int T>
+__global__ void __launch_bounds__(T)
+    verify_part_kernel(const float* logits, int V, int span, int n_parts, uint32_t* greedy) {
+  __shared__ uint64_t red[T / 64];
+  const uint32_t r = blockIdx.x / (uint32_t)n_parts;
+  const int i0 = (int)(blockIdx.x % (uint32_t)n_parts) * span;
+  const float* x = logits + (int64_t)r * V;
+  uint32_t cur = 0u;
+  if (threadIdx.x == 0) cur = __hip_atomic_load(greedy + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  float xc = -__builtin_inff();
+  const uint64_t best = verify_span_max<T>(x, V, i0, min(i0 + span, V), red, [&]() {
+    if (cur < (uint32_t)V && threadIdx.x == 0) xc = x[cur];
+  });
+  if (threadIdx.x == 0 && best != 0ull) verify_take(x, V, best, cur, xc, greedy + r);
 }
 
-// greedy[r] by one workgroup a row, for a call that cannot have the parts'
-// buffer.
-__global__ void __launch_bounds__(kVerifyThreads) verify_argmax_kernel(const float* logits, int V, uint32_t* greedy) {
-  __shared__ uint64_t red[kVerifyThreads / 64];
-  const float* x = logits + (int64_t)blockIdx.x * V;
-  const uint64_t best = verify_span_max(x, V, 0, V, red);
-  if (threadIdx.x == 0) greedy[blockIdx.x] = verify_index(best, x[0]);
-}
-
-// One workgroup per request: its rows' greedy tokens from their parts (a
-// wave a row, n_parts <= 64; null: greedy holds them already), the accepted
-// prefix and the emitted tokens.
-__global__ void __launch_bounds__(kVerifyThreads)
-    verify_accept_kernel(const float* logits, int V, const uint64_t* parts, int n_parts, uint32_t* greedy,
-                         const uint32_t* draft, const int32_t* draft_len, int K, uint32_t* out_tokens,
-                         int32_t* out_count) {
+constexpr int kAcceptThreads = 256;
+// One workgroup per request: its rows' answers (index 0 with a NaN there, or
+// when nothing is above -inf), the accepted prefix and the emitted tokens.
+__global__ void __launch_bounds__(kAcceptThreads)
+    verify_accept_kernel(const float* logits, int V, uint32_t* greedy, const uint32_t* draft, const int32_t* draft_len,
+                         int K, uint32_t* out_tokens, int32_t* out_count) {
   __shared__ int accepted;
-  const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int b = blockIdx.x, tid = threadIdx.x;
   const int64_t r0 = (int64_t)b * (K + 1);
   const int k = draft_len ? min(max(draft_len[b], 0), K) : K;
   if (tid == 0) accepted = k;
-  if (parts) {
-    for (int i = tid >> 6; i <= K; i += kVerifyThreads / 64) {
-      const float x0 = logits[(r0 + i) * V];
-      const uint64_t best = verify_wave_max(lane < n_parts ? parts[(r0 + i) * n_parts + lane] : 0ull);
-      if (lane == 0) greedy[r0 + i] = verify_index(best, x0);
-    }
+  __syncthreads();
+  for (int i = tid; i <= K; i += kAcceptThreads) {
+    const float* x = logits + (r0 + i) * V;
+    uint32_t g = greedy[r0 + i];
+    const float x0 = x[0], xg = g < (uint32_t)V ? x[g] : -__builtin_inff();
+    if (x0 != x0 || !(xg > -__builtin_inff())) greedy[r0 + i] = g = 0u;
+    if (i < k && draft[(int64_t)b * K + i] != g) atomicMin(&accepted, i);
   }
   __syncthreads();
-  for (int i = tid; i < k; i += kVerifyThreads)
-    if (draft[(int64_t)b * K + i] != greedy[r0 + i]) atomicMin(&accepted, i);
-  __syncthreads();
   const int n = accepted;
-  for (int i = tid; i <= n; i += kVerifyThreads) out_tokens[r0 + i] = greedy[r0 + i];
+  for (int i = tid; i <= n; i += kAcceptThreads) out_tokens[r0 + i] = greedy[r0 + i];
   if (tid == 0) out_count[b] = n + 1;
 }
 
-// Parts of a row: steps of kVerifySpan logits, at most 64 (a wave merges
-// them).  One step a workgroup fills the chip from a few rows on (40 rows of
-// 151,936: 760 workgroups, 61.7 -> 9.0 us).
+// Parts of a row: steps of kVerifySpan logits, at most 64.  Rows of one step
+// of 256 threads take such workgroups, longer ones steps of 1024: the parts
+// of a row exchange through the memory behind the chip's L2s, about 5 ns an
+// exchange on one cache line, so larger parts win from the first row that is
+// split (40 rows of 151,936: 10.3 us, in parts of 256 threads 15.6, in one
+// workgroup a row 12.7; 264 rows: 33, 42 and 40; 4096 rows of 4096: 14.4
+// with 256 threads, 34 with 1024).  One workgroup of 1024 threads a row, with
+// one load a thread in flight, took 62 us for the 40 rows.  A grid holds less
+// than 2^32 work-items, so many rows take fewer parts.  (Inputs that change
+// from call to call; answers that the array already holds exchange nothing.)
 constexpr int kVerifyMaxParts = 64;
-std::mutex g_verify_mutex;  // both launches of a call on a stream's buffer, together
+
+template <int T>
+void launch_parts(const float* x, int64_t rows, int V, uint32_t* greedy, hipStream_t st) {
+  constexpr int64_t kMaxGroups = (((int64_t)1 << 32) - 1) / T;
+  const int steps = (V + kVerifySpan<T> - 1) / kVerifySpan<T>;
+  const int most = (int)std::min<int64_t>(kVerifyMaxParts, std::max<int64_t>(1, kMaxGroups / rows));
+  const int span = kVerifySpan<T> * ((steps + most - 1) / most);
+  const int n_parts = (V + span - 1) / span;
+  hipLaunchKernelGGL((verify_part_kernel<T>), dim3((unsigned)(rows * n_parts)), dim3(T), 0, st, x, V, span, n_parts,
+                     greedy);
+}
 
 }  // namespace
 }  // namespace hi_rocm
@@ -159,27 +193,15 @@ extern "C" int hi_rocm_spec_verify_greedy(const void* logits, int batch, int max
   if (rows > INT32_MAX) return hi_rocm::api_fail(HI_ROCM_ERR_UNSUPPORTED, "hi_rocm_spec_verify_greedy: too many rows");
   hipStream_t st = (hipStream_t)stream;
   namespace hr = hi_rocm;
-  const int steps = (vocab + hr::kVerifySpan - 1) / hr::kVerifySpan;
-  const int span = hr::kVerifySpan * ((steps + hr::kVerifyMaxParts - 1) / hr::kVerifyMaxParts);
-  const int n_parts = (vocab + span - 1) / span;
   const float* x = (const float*)logits;
   uint32_t* greedy = (uint32_t*)out_greedy;
-  std::lock_guard<std::mutex> lock(hr::g_verify_mutex);
-  // the stream's buffer for the parts; none while a capture would have to
-  // allocate it, or beyond a grid's rows: then one workgroup a row
-  void* ws = nullptr;
-  if (rows <= 65535) {
-    const int rc = hr::api_stream_buffer(hr::kWsVerify, (size_t)rows * n_parts * sizeof(uint64_t), 0, true, st, &ws);
-    if (rc != HI_ROCM_OK) return rc;
-  }
-  if (ws)
-    hipLaunchKernelGGL(hr::verify_part_kernel, dim3((unsigned)n_parts, (unsigned)rows), dim3(hr::kVerifyThreads), 0, st,
-                       x, vocab, span, (uint64_t*)ws);
+  if (vocab <= hr::kVerifySpan<256>)
+    hr::launch_parts<256>(x, rows, vocab, greedy, st);
   else
-    hipLaunchKernelGGL(hr::verify_argmax_kernel, dim3((unsigned)rows), dim3(hr::kVerifyThreads), 0, st, x, vocab, greedy);
-  hipLaunchKernelGGL(hr::verify_accept_kernel, dim3((unsigned)batch), dim3(hr::kVerifyThreads), 0, st, x, vocab,
-                     (const uint64_t*)ws, n_parts, greedy, (const uint32_t*)draft_tokens, (const int32_t*)draft_len,
-                     max_draft, (uint32_t*)out_tokens, (int32_t*)out_count);
+    hr::launch_parts<1024>(x, rows, vocab, greedy, st);
+  hipLaunchKernelGGL(hr::verify_accept_kernel, dim3((unsigned)batch), dim3(hr::kAcceptThreads), 0, st, x, vocab, greedy,
+                     (const uint32_t*)draft_tokens, (const int32_t*)draft_len, max_draft, (uint32_t*)out_tokens,
+                     (int32_t*)out_count);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? HI_ROCM_OK : hr::api_hip_fail(e, "spec verify launch");
 }

@@ -55,14 +55,50 @@ def test_spec_verify_parity(hip, oracle, B, K, V):
             assert (tt[b, cc[b]:] == 0xffffffff).all(), "write past the emitted tokens"
 
 
+def _stream_of_its_own(torch):
+    """A new stream and its handle (torch's come from a pool)."""
+    handle = ctypes.c_uint64()
+    assert int(torch.cuda.cudart().cudaStreamCreate(ctypes.addressof(handle))) == 0
+    return torch.cuda.ExternalStream(handle.value), handle
+
+
+class _Call:
+    """One verification's device arrays and what the oracle says of them."""
+
+    def __init__(self, torch, oracle, x, d):
+        self.want = oracle.spec_verify_greedy(x, d, None)
+        self.B, self.K, self.V = x.shape[0], x.shape[1] - 1, x.shape[2]
+        self.x, self.d = torch.from_numpy(x).cuda(), torch.from_numpy(d.view(np.int32)).cuda()
+        self.g, self.t = (torch.full((self.B, self.K + 1), -1, dtype=torch.int32, device="cuda") for _ in range(2))
+        self.c = torch.full((self.B,), -1, dtype=torch.int32, device="cuda")
+
+    def launch(self, hip, handle):
+        hip.check(hip.load().hi_rocm_spec_verify_greedy(
+            self.x.data_ptr(), self.B, self.K, self.V, self.d.data_ptr(), 0, self.g.data_ptr(), self.t.data_ptr(),
+            self.c.data_ptr(), handle))
+
+    def clear(self, greedy=-1):
+        for o in (self.g, self.t, self.c):
+            o.fill_(-1)
+        self.g.fill_(greedy)
+
+    def same(self):
+        wg, wt, wc = self.want
+        assert np.array_equal(self.g.cpu().numpy().view(np.uint32), wg)
+        assert np.array_equal(self.c.cpu().numpy(), wc)
+        t = self.t.cpu().numpy().view(np.uint32)
+        assert all(np.array_equal(t[b, :wc[b]], wt[b, :wc[b]]) for b in range(self.B))
+        assert all((t[b, wc[b]:] == 0xffffffff).all() for b in range(self.B)), "write past the emitted tokens"
+
+
 @pytest.mark.parametrize("V", [1, 8191, 8193, 50257, 70001])
 def test_spec_verify_parts(hip, oracle, V):
-    """Rows split over workgroups (8192 logits each) and, inside a capture
-    whose stream has no buffer yet, one workgroup a row: maxima on both
-    sides of every part's edge, equal maxima in two parts, -inf and NaN
-    rows; the capture replayed three times."""
+    """Rows split over workgroups (8192 logits each), eagerly and in a capture
+    on a stream of no earlier call: maxima on both sides of every part's edge,
+    equal maxima in two parts, -inf and NaN rows, and whatever the greedy
+    array holds before: no index, one past the row, a NaN's, an equal maximum
+    that is not the first."""
     import torch
-    lib = hip.load()
     B, K = 6, 2
     rng = np.random.default_rng(V)
     x = (rng.standard_normal((B, K + 1, V)) * 2).astype(F32)
@@ -70,46 +106,75 @@ def test_spec_verify_parts(hip, oracle, V):
     for n, e in enumerate(edges):
         x[n % B, n % (K + 1), e] = 50.0
     x[4, 0, edges] = 60.0
+    x[4, 1, :] = 0.0
+    x[4, 1, ::2] = -0.0
     x[5, 0, :] = -np.inf
     x[5, 1, :] = np.nan
     x[5, 2, V // 2:] = np.nan
     d = rng.integers(0, V, (B, K)).astype(np.uint32)
-    wg, wt, wc = oracle.spec_verify_greedy(x, d, None)
-    d[:, 0] = wg[:, 0]
-    wg, wt, wc = oracle.spec_verify_greedy(x, d, None)
-    dx, dd = torch.from_numpy(x).cuda(), torch.from_numpy(d.view(np.int32)).cuda()
-    g, t = (torch.full((B, K + 1), -1, dtype=torch.int32, device="cuda") for _ in range(2))
-    c = torch.full((B,), -1, dtype=torch.int32, device="cuda")
-
-    def call(s):
-        hip.check(lib.hi_rocm_spec_verify_greedy(dx.data_ptr(), B, K, V, dd.data_ptr(), 0, g.data_ptr(), t.data_ptr(),
-                                                 c.data_ptr(), s.cuda_stream))
-
-    def same():
-        assert np.array_equal(g.cpu().numpy().view(np.uint32), wg)
-        assert np.array_equal(c.cpu().numpy(), wc)
-        tt = t.cpu().numpy().view(np.uint32)
-        assert all(np.array_equal(tt[b, :wc[b]], wt[b, :wc[b]]) for b in range(B))
-
-    handle = ctypes.c_uint64()  # a stream of its own: torch's come from a pool and may already hold a buffer
-    assert int(torch.cuda.cudart().cudaStreamCreate(ctypes.addressof(handle))) == 0
-    s = torch.cuda.ExternalStream(handle.value)
+    d[:, 0] = oracle.spec_verify_greedy(x, d, None)[0][:, 0]
+    call = _Call(torch, oracle, x, d)
+    s, handle = _stream_of_its_own(torch)
     torch.cuda.synchronize()
     print(f"spec verify parts V={V}", flush=True)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph, stream=s):
-        call(s)
-    for _ in range(3):
-        g.fill_(-1)
+        call.launch(hip, s.cuda_stream)
+    for before in (-1, 0, V, V - 1, V // 2):
+        call.clear(before)
         graph.replay()
         torch.cuda.synchronize()
-        same()
-    for _ in range(2):
-        g.fill_(-1)
+        call.same()
+        call.clear(before)
         torch.cuda.synchronize()
-        call(s)
+        call.launch(hip, s.cuda_stream)
         s.synchronize()
-        same()
-    hip.check(lib.hi_rocm_sampler_release(s.cuda_stream))
+        call.same()
     del graph, s
+    assert int(torch.cuda.cudart().cudaStreamDestroy(handle.value)) == 0
+
+
+def test_spec_verify_calls_share_nothing(hip, oracle):
+    """Calls with different outputs at once: two graphs captured on one stream
+    and replayed on two others, beside eager calls on the capture stream, each
+    checked after every round; releasing the stream's library buffers leaves
+    the graphs whole, and no call allocates."""
+    import torch
+    B, K, V = 8, 4, 151936
+    calls = []
+    for seed in range(3):
+        rng = np.random.default_rng(seed)
+        x = rng.standard_normal((B, K + 1, V), dtype=F32)
+        d = x[:, :K].argmax(2).astype(np.uint32)
+        d[::3, seed] += 1
+        calls.append(_Call(torch, oracle, x, d))
+    s, handle = _stream_of_its_own(torch)
+    others = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for c in calls:  # the kernels' first launches
+        c.launch(hip, others[0].cuda_stream)
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    calls[2].launch(hip, s.cuda_stream)  # the stream's first call
+    torch.cuda.synchronize()
+    assert torch.cuda.mem_get_info()[0] == free0, "a verification allocated"
+    graphs = []
+    for c in calls[:2]:
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1], stream=s):
+            c.launch(hip, s.cuda_stream)
+    hip.check(hip.load().hi_rocm_sampler_release(s.cuda_stream))
+    print("spec verify: concurrent calls", flush=True)
+    for _ in range(20):
+        for c in calls:
+            c.clear()
+        torch.cuda.synchronize()
+        for _ in range(3):
+            for graph, o in zip(graphs, others):
+                with torch.cuda.stream(o):
+                    graph.replay()
+            calls[2].launch(hip, s.cuda_stream)
+        torch.cuda.synchronize()
+        for c in calls:
+            c.same()
+    del graphs, s
     assert int(torch.cuda.cudart().cudaStreamDestroy(handle.value)) == 0
