@@ -55,37 +55,39 @@ __device__ __forceinline__ uint64_t verify_wave_max(uint64_t best) {
   return best;
 }
 
-// The key of the row's first maximum above -inf in [i0, i1) (0: none), by a
-// workgroup of T threads: range-checked 16-byte loads, kVerifyLoads a thread
-// in flight.  ahead() is called behind the first ones.
+// The key of the first maximum above -inf of the row x in [i0, i0 + n) (0:
+// none), by a workgroup of T threads: range-checked 16-byte loads,
+// kVerifyLoads a thread in flight, from a buffer of the part's own (ranges
+// and offsets count bytes in 32 bits).  ahead() is called behind the first
+// ones.
 constexpr int kVerifyLoads = 8;
 template <int T>
 constexpr int kVerifySpan = T * 4 * kVerifyLoads;  // logits of a step
 template <int T, typename AheadF>
-__device__ __forceinline__ uint64_t verify_span_max(const float* x, int V, int i0, int i1, uint64_t* red, AheadF ahead) {
+__device__ __forceinline__ uint64_t verify_span_max(const float* x, int64_t i0, int n, uint64_t* red, AheadF ahead) {
   const int tid = threadIdx.x;
-  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, V * 4, kBufferConfig);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(x + i0), 0, n * 4, kBufferConfig);
   float bv = -__builtin_inff();
   uint32_t bi = 0xffffffffu;
-  for (int b = i0; b < i1; b += kVerifySpan<T>) {
+  for (int b = 0; b < n; b += kVerifySpan<T>) {
     i32x4_t v[kVerifyLoads];
     #pragma unroll
     for (int j = 0; j < kVerifyLoads; ++j)
       v[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, (b + (j * T + tid) * 4) * 4, 0, 0);
-    if (b == i0) ahead();
+    if (b == 0) ahead();
     #pragma unroll
     for (int j = 0; j < kVerifyLoads; ++j) {
       #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int i = b + (j * T + tid) * 4 + q;
         const float f = __int_as_float(v[j][q]);
-        const bool take = f > bv && i < V;  // (NaN never; a thread's indices rise)
+        const bool take = f > bv && i < n;  // (NaN never; a thread's indices rise)
         bv = take ? f : bv;
         bi = take ? (uint32_t)i : bi;
       }
     }
   }
-  uint64_t best = verify_wave_max(bi == 0xffffffffu ? 0ull : verify_key(bv, bi));
+  uint64_t best = verify_wave_max(bi == 0xffffffffu ? 0ull : verify_key(bv, (uint32_t)i0 + bi));
   if ((tid & 63) == 0) red[tid >> 6] = best;
   __syncthreads();
   best = red[0];
@@ -121,12 +123,12 @@ __global__ void __launch_bounds__(T)
     verify_part_kernel(const float* logits, int V, int span, int n_parts, uint32_t* greedy) {
   __shared__ uint64_t red[T / 64];
   const uint32_t r = blockIdx.x / (uint32_t)n_parts;
-  const int i0 = (int)(blockIdx.x % (uint32_t)n_parts) * span;
+  const int64_t i0 = (int64_t)(blockIdx.x % (uint32_t)n_parts) * span;
   const float* x = logits + (int64_t)r * V;
   uint32_t cur = 0u;
   if (threadIdx.x == 0) cur = __hip_atomic_load(greedy + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   float xc = -__builtin_inff();
-  const uint64_t best = verify_span_max<T>(x, V, i0, min(i0 + span, V), red, [&]() {
+  const uint64_t best = verify_span_max<T>(x, i0, (int)min((int64_t)span, V - i0), red, [&]() {
     if (cur < (uint32_t)V && threadIdx.x == 0) xc = x[cur];
   });
   if (threadIdx.x == 0 && best != 0ull) verify_take(x, V, best, cur, xc, greedy + r);
@@ -172,10 +174,11 @@ constexpr int kVerifyMaxParts = 64;
 template <int T>
 void launch_parts(const float* x, int64_t rows, int V, uint32_t* greedy, hipStream_t st) {
   constexpr int64_t kMaxGroups = (((int64_t)1 << 32) - 1) / T;
-  const int steps = (V + kVerifySpan<T> - 1) / kVerifySpan<T>;
-  const int most = (int)std::min<int64_t>(kVerifyMaxParts, std::max<int64_t>(1, kMaxGroups / rows));
-  const int span = kVerifySpan<T> * ((steps + most - 1) / most);
-  const int n_parts = (V + span - 1) / span;
+  const int64_t steps = ((int64_t)V + kVerifySpan<T> - 1) / kVerifySpan<T>;
+  const int64_t most = std::min<int64_t>(kVerifyMaxParts, std::max<int64_t>(1, kMaxGroups / rows));
+  // (2^28 logits are 2^30 bytes; with 64 parts a row's part is at most 2^25)
+  const int span = (int)std::min<int64_t>(kVerifySpan<T> * ((steps + most - 1) / most), 1 << 28);
+  const int n_parts = (int)((V + (int64_t)span - 1) / span);
   hipLaunchKernelGGL((verify_part_kernel<T>), dim3((unsigned)(rows * n_parts)), dim3(T), 0, st, x, V, span, n_parts,
                      greedy);
 }

@@ -178,3 +178,23 @@ def test_spec_verify_calls_share_nothing(hip, oracle):
             c.same()
     del graphs, s
     assert int(torch.cuda.cudart().cudaStreamDestroy(handle.value)) == 0
+
+
+def test_spec_verify_beyond_32_bit_bytes(hip):
+    """A row of more than 2^32 bytes: the maximum is found wherever it lies,
+    and of two equal ones the first."""
+    import torch
+    lib = hip.load()
+    V = 2 ** 30 + 5
+    x = torch.full((V,), -1.0, device="cuda")
+    d, g, t, c = (torch.zeros(2, dtype=torch.int32, device="cuda") for _ in range(4))
+    st = torch.cuda.Stream()
+    for at in ([3], [2 ** 29 - 1, 2 ** 29 + 3], [2 ** 29 + 3], [2 ** 30 - 1, 2 ** 30 + 2], [2 ** 30 + 2], [V - 1]):
+        x[at] = 2.0
+        torch.cuda.synchronize()
+        print(f"spec verify V={V} {at}", flush=True)
+        hip.check(lib.hi_rocm_spec_verify_greedy(x.data_ptr(), 1, 0, V, 0, 0, g.data_ptr(), t.data_ptr(), c.data_ptr(),
+                                                 st.cuda_stream))
+        torch.cuda.synchronize()
+        assert (int(g[0]), int(t[0]), int(c[0])) == (at[0], at[0], 1)
+        x[at] = -1.0
