@@ -5,6 +5,9 @@
 
 namespace hi_rocm {
 
+constexpr int kCus = 256;
+static_assert(kFusedMaxWorkgroups == 2 * kCus, "two workgroups a CU");
+
 // The streaming select pass and the finish in one launch, for small
 // batches: the last workgroup of a row to finish its chunk (a device-scope
 // counter per row) runs the row's finish.  The other workgroups' records
@@ -12,11 +15,21 @@ namespace hi_rocm {
 // acquired by the last one's fence after it (one thread fences for the
 // workgroup, between barriers); the last one also sets the counter back to
 // zero for the next launch.  No workgroup waits for another.
+// Two workgroups a CU: FinLds lets two share one, and the registers are held
+// to that (at 268 of them one workgroup filled a CU: 12 rows of 151,936, 456
+// workgroups, took 20.3 us greedy and 28.6 top-k; now 16.6 and 25.9).
+// Workgroups i and i + kCus land on one CU as the dispatcher goes round, so
+// they are neighbours in one row: two rows' finishes on one CU share its
+// SIMDs, and those CUs also end last (the 12 rows by nucleus: 405 us, 488
+// with a row's workgroups in the grid's order).
 template <int DT, int NL, bool MASK>
-__global__ void __launch_bounds__(NT) select_finish_kernel(SampleArgs a, uint32_t flag_off) {
+__global__ void __launch_bounds__(NT, kFusedMaxWorkgroups / kCus) select_finish_kernel(SampleArgs a, uint32_t flag_off) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  const int row = blockIdx.y;
-  select_chunk<DT, NL, MASK>(a, row, blockIdx.x, lds_raw);
+  // workgroup i's place in the order of (i % kCus, i / kCus)
+  const int over = max((int)gridDim.x - kCus, 0), i = blockIdx.x;
+  const int place = i < kCus ? i + min(i, over) : 2 * (i - kCus) + 1;
+  const int row = place / a.n_chunks;
+  select_chunk<DT, NL, MASK>(a, row, place % a.n_chunks, lds_raw);
   uint32_t* last = reinterpret_cast<uint32_t*>(lds_raw + flag_off);  // past both LDS layouts
   // every wave waits for its stores to reach L2 (a workgroup barrier alone
   // does not), then one device-scope fence writes them back before the
@@ -54,7 +67,7 @@ hipError_t launch_fused_t(const SampleArgs& a, hipStream_t stream) {
   const size_t lds = body + 16;
   hipError_t e = ensure_lds((const void*)select_finish_kernel<DT, NL, MASK>, lds);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((select_finish_kernel<DT, NL, MASK>), dim3(a.n_chunks, a.B), dim3(NT), lds, stream, a,
+  hipLaunchKernelGGL((select_finish_kernel<DT, NL, MASK>), dim3(a.n_chunks * a.B), dim3(NT), lds, stream, a,
                      (uint32_t)body);
   return hipGetLastError();
 }

@@ -110,3 +110,25 @@ def test_row_kernel_other_classes(hip, oracle, with_mask, V):
     got = out["tokens"].cpu().numpy().view(np.uint32)
     bad = np.flatnonzero(got != want)
     assert bad.size == 0, (bad, got[bad], want[bad])
+
+
+@pytest.mark.parametrize("B,V", [(256, 4096), (257, 100), (129, 4097), (37, 33001), (512, 257), (12, 151936), (2, 1048575)])
+def test_one_launch_grids(hip, oracle, B, V):
+    """Grids of 256 to 512 workgroups (4096 logits each), whose workgroups
+    are dealt to the rows by CU: every row class, tokens equal the oracle's."""
+    import torch
+    from hi_amd import sampler as S
+    x = _rows("spiked", B, V, B + V)
+    p = _params(B)
+    p["temperature"][0::7] = 0.0
+    p["top_k"][1::6] = 40
+    u = np.random.default_rng(B).random(B).astype(F32)
+    smp = S.Sampler(B, V)
+    print(f"one launch B={B} V={V}", flush=True)
+    for _ in range(2):
+        out = smp.sample(torch.from_numpy(x).cuda(), S.params_to_device(p), torch.from_numpy(u).cuda())
+        torch.cuda.synchronize()
+        got = out["tokens"].cpu().numpy().view(np.uint32)
+        want = oracle.sample_rows(x, p, u)["tokens"]
+        bad = np.flatnonzero(got != want)
+        assert bad.size == 0, (bad, got[bad], want[bad])
