@@ -55,20 +55,25 @@ __global__ void __launch_bounds__(NT) finish_kernel(SampleArgs a) {
 // else finish_row) and its other workgroups exit at once.  Workgroups go to
 // the XCDs and their shader engines round-robin by linear id, so the B
 // finishing workgroups, being consecutive, spread over the whole chip (on a
-// (chunks, rows) grid they would share a few engines).
+// (chunks, rows) grid they would share a few engines).  The rest take an odd
+// number of places a row: at a multiple of 8 every row's last unit, which
+// finishes it, and the working units of a temperature-only row would land on
+// the same XCDs (64 rows of 262,208: nucleus 878 -> 813 us, min-p 417 -> 385,
+// temperature only 144 -> 89).
 __global__ void __launch_bounds__(NT) finish_grid_kernel(SampleArgs a, WideUnits wu) {
   extern __shared__ __align__(16) unsigned char lds_raw[];
   int row = (int)blockIdx.x, unit = 0;
   if (row >= a.B) {
-    const int rest = row - a.B, per = wu.n - 1;
+    const int rest = row - a.B, per = (wu.n - 1) | 1;
     row = rest / per;
     unit = 1 + rest % per;
+    if (unit >= wu.n) return;
   }
   const RowCfg cfg = load_cfg(a.pv, row, a.V, a.n_lp, a.need_lse);
   FinLds& fs = *reinterpret_cast<FinLds*>(lds_raw);
   // (the reference chunks' sums of a temperature-only row need 256 floats of
   // its ws_list)
-  const bool wide = wide_fits(a) &&
+  const bool wide = wide_fits(wu) &&
                     (cfg.cls == kTopP || (cfg.cls == kTempOnly && a.list_stride >= 128 && wu.n >= kTempSplit && a.B <= kTempRows));
   if (!wide) {
     if (unit != 0) return;
@@ -80,7 +85,7 @@ __global__ void __launch_bounds__(NT) finish_grid_kernel(SampleArgs a, WideUnits
   const int parts = cfg.cls == kTopP ? wu.n : kTempSplit;  // workgroups of the row that work
   if (unit >= parts) return;
   WideChunkLds& L = *reinterpret_cast<WideChunkLds*>(lds_raw);
-  const DrawRow r = draw_row<NT>(a, row);
+  const DrawRow r = wide_row(a, row);
   bool valid;
   float M, w_lo = 0.f;
   if (cfg.cls == kTopP) {
@@ -217,7 +222,7 @@ hipError_t launch_sample(const SampleArgs& a, hipStream_t stream, const LaunchEv
   if (e == hipSuccess) e = record(le, 1, stream);
   if (e != hipSuccess) return e;
   const WideUnits wu = wide_units(a.B, a.V, a.chunk, a.n_chunks);
-  const int64_t n_wg = (int64_t)wu.n * a.B;
+  const int64_t n_wg = (int64_t)(1 + ((wu.n - 1) | 1)) * a.B;
   if (n_wg * NT >= ((int64_t)1 << 32)) return hipErrorInvalidConfiguration;  // 1-D grid of work-items
   const size_t lds = finish_grid_lds();
   e = ensure_lds((const void*)finish_grid_kernel, lds);

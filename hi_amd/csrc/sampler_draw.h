@@ -371,14 +371,13 @@ __device__ __forceinline__ void draw_collect(DrawLds<NTH>& D, const float* tr, c
     if (at < (uint32_t)kDrawPiece) D.u.p.key0[at] = top - __float_as_uint(tr[lane * kTrLd + __ffs((int)mk) - 1]);
 }
 
-// The chain over the row's tiles from -0.0 (wave 0, lane l holding tile tb +
-// l), to D.total: scans over the tiles of one binade, exact folds of the
-// others.
+// The chain from `acc` over the row's tiles t0, ..., t0 + nt - 1, whose maps D
+// holds (wave 0, lane l holding tile t0 + tb + l), to D.total: scans over the
+// tiles of one binade, exact folds of the others.
 template <int NTH>
-__device__ __forceinline__ void draw_chain(DrawLds<NTH>& D, const DrawRow& r, int nt) {
+__device__ __forceinline__ void draw_chain(DrawLds<NTH>& D, const DrawRow& r, int t0, int nt, float acc) {
   const int lane = (int)(threadIdx.x & 63u);
   const int span = 64 * kDrawPer * r.mult;
-  float acc = -0.0f;
   for (int tb = 0; tb < nt; tb += 64) {
     const int n = min(64, nt - tb);
     const uint32_t bin = lane < n ? D.tbin[tb + lane] : 0u;
@@ -399,7 +398,7 @@ __device__ __forceinline__ void draw_chain(DrawLds<NTH>& D, const DrawRow& r, in
       if (f < n) {
         for (int g = 0; g < r.mult; ++g) {
           float x[kDrawPer];
-          draw_lane_terms(r, (tb + f) * span + g * 64 * kDrawPer, x);
+          draw_lane_terms(r, (t0 + tb + f) * span + g * 64 * kDrawPer, x);
           acc = wave_fold_blocks(x, acc, [](float) {});
         }
       }
@@ -438,7 +437,7 @@ __device__ __forceinline__ void draw_total(DrawLds<NTH>& D, const DrawRow& r, ui
     }
   });
   __syncthreads();
-  if (wid == 0) draw_chain<NTH>(D, r, nt);
+  if (wid == 0) draw_chain<NTH>(D, r, 0, nt, -0.0f);
   __syncthreads();
 }
 

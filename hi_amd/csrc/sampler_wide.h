@@ -30,7 +30,7 @@ namespace hi_rocm {
 // A temperature-only row's workgroups sum its 256 reference chunks instead,
 // one wave a chunk, and the last one draws.
 // Rows whose chunks took the select pass's exact path, whose nucleus is not
-// inside the listed weights, or of more than 256 tiles take finish_row.
+// inside the listed weights, or of more than 256 units take finish_row.
 //
 // A workgroup takes a unit of one or several select chunks (WideUnits): every
 // workgroup of a row repeats the row statistics (about 5 us), so once the
@@ -65,7 +65,7 @@ struct WideUnits {
 __host__ __device__ inline WideUnits wide_units(int B, int V, int chunk, int n_chunks) {
   // 64 nucleus rows of 151,936: 192 us with units of one chunk, 122 us
   // with units of four; 32 masked rows: 107 and 86 us
-  const int g = chunk < kSelChunkLarge && (int64_t)B * n_chunks > 768 ? kSelChunkLarge / chunk : 1;
+  const int g = chunk < kSelChunkLarge && ((int64_t)B * n_chunks > 768 || n_chunks > kDrawChunks) ? kSelChunkLarge / chunk : 1;
   return WideUnits{(n_chunks + g - 1) / g, chunk * g, g};
 }
 
@@ -114,7 +114,8 @@ __device__ __forceinline__ uint32_t wide_hash(uint32_t key, int log2n) {
 // Inserts `count` copies of weight bits `key` with smallest index `idx`
 // into an LDS table of 2^log2n slots (key 0 = empty; weights here are > 0).
 // Returns false when kWideProbes slots in a row hold other weights (a table
-// that fills up would otherwise be searched end to end for every weight).
+// that fills up would otherwise be searched end to end for every weight); a
+// thread inserts nothing more then.
 __device__ __forceinline__ bool wide_insert(uint32_t* hkey, uint32_t* hcnt, uint32_t* hmin, int log2n,
                                             uint32_t key, uint32_t count, uint32_t idx) {
   const uint32_t mask = (1u << log2n) - 1u;
@@ -347,9 +348,9 @@ __device__ __forceinline__ void wide_chunk_work(WideChunkLds& L, const SampleArg
     for (int q = 0; q < kDrawPer; ++q) mk |= x[i][q] > 0.f && x[i][q] >= w_lo ? 1u << q : 0u;
     if (__ballot(mk != 0u) == 0ull) continue;
     if (runs) {
-      for (; mk != 0u; mk &= mk - 1u) {
+      for (; mk != 0u && !full; mk &= mk - 1u) {
         const int q = __ffs((int)mk) - 1;
-        full |= !wide_insert(L.hkey, L.hcnt, L.hmin, kWideLog2, __float_as_uint(tr[lane * kTrLd + q]), 1u,
+        full = !wide_insert(L.hkey, L.hcnt, L.hmin, kWideLog2, __float_as_uint(tr[lane * kTrLd + q]), 1u,
                              (uint32_t)(t0 - c0 + lane * kDrawPer + q));
       }
       continue;
@@ -545,8 +546,8 @@ __device__ __forceinline__ uint32_t wide_finish_runs(WideRunLds& F, const Sample
   __syncthreads();
   bool full = false;
   auto insert = [&](int c, uint64_t e) {
-    full |= !wide_insert(F.u.mg.hkey, F.u.mg.hcnt, F.u.mg.hmin, kWideLog2, (uint32_t)(e >> 32),
-                         (uint32_t)(e >> 16) & 0xffffu, (uint32_t)(c * wu.len) + ((uint32_t)e & 0xffffu));
+    if (!full) full = !wide_insert(F.u.mg.hkey, F.u.mg.hcnt, F.u.mg.hmin, kWideLog2, (uint32_t)(e >> 32),
+                                   (uint32_t)(e >> 16) & 0xffffu, (uint32_t)(c * wu.len) + ((uint32_t)e & 0xffffu));
   };
   wide_for_each_run(F, a, row, wu, (int)n_all, insert);
   path = kWideNoCutoff;
@@ -749,9 +750,14 @@ __device__ __forceinline__ uint32_t wide_finish_runs(WideRunLds& F, const Sample
   return F.tok;
 }
 
-// Whether the wide pass takes the row: its tiles and chunks fit the tables.
-__device__ __forceinline__ bool wide_fits(const SampleArgs& a) {
-  return a.V <= kDrawTiles * kWideTile && a.n_chunks <= kDrawChunks;
+// Whether the wide pass takes the rows: their units fit the tables (up to
+// 4,194,304 logits in units of 16,384).  The row of its tiles, whose maps are
+// chained kDrawTiles at a time.
+__device__ __forceinline__ bool wide_fits(const WideUnits& wu) { return wu.n <= kDrawChunks; }
+__device__ __forceinline__ DrawRow wide_row(const SampleArgs& a, int row) {
+  DrawRow r = draw_row<NT>(a, row);
+  r.mult = 1;
+  return r;
 }
 
 // Step 4: the finish of a top-p row by its last workgroup.  Returns the
@@ -767,12 +773,15 @@ __device__ __forceinline__ uint32_t wide_finish(DrawLds<NT>& D, const SampleArgs
   const uint32_t cn = tid < nch ? folds[tid].n : 0u;
   const bool ovf = __syncthreads_or(cn == kFoldNone);
   const uint32_t mine = ovf ? 0u : cn;
-  if (tid < nt) {
-    const ChunkFold& f = folds[tid / per];
-    D.tmap[tid] = f.map[tid % per];
-    D.tlow[tid] = f.low[tid % per];
-    D.tbin[tid] = f.bin[tid % per];
-  }
+  auto load_tiles = [&](int t0) {
+    if (t0 + tid < nt) {
+      const ChunkFold& f = folds[(t0 + tid) / per];
+      D.tmap[tid] = f.map[(t0 + tid) % per];
+      D.tlow[tid] = f.low[(t0 + tid) % per];
+      D.tbin[tid] = f.bin[(t0 + tid) % per];
+    }
+  };
+  load_tiles(0);
   for (int b = tid; b < kDrawBins + kDrawBins / 32; b += NT) D.hist[b] = 0u;
   uint32_t n_all;
   D.noff[tid] = block_excl_scan_u32<NT>(mine, D.red, &n_all);
@@ -786,7 +795,7 @@ __device__ __forceinline__ uint32_t wide_finish(DrawLds<NT>& D, const SampleArgs
   const bool one = n_all <= (uint32_t)kDrawPiece;  // every listed weight fits a piece
   constexpr uint32_t kTop = (uint32_t)((kDrawAll - 1u) >> 23);
   if (wid == 0) {
-    draw_chain<NT>(D, r, nt);
+    draw_chain<NT>(D, r, 0, min(nt, kDrawTiles), -0.0f);
   } else if (runs) {
   } else if (one) {
     int p = tid - 64;  // entries in order: p, p + 192, ...
@@ -800,6 +809,12 @@ __device__ __forceinline__ uint32_t wide_finish(DrawLds<NT>& D, const SampleArgs
     });
   }
   __syncthreads();
+  for (int t0 = kDrawTiles; t0 < nt; t0 += kDrawTiles) {
+    load_tiles(t0);
+    __syncthreads();
+    if (wid == 0) draw_chain<NT>(D, r, t0, min(nt - t0, kDrawTiles), D.total);
+    __syncthreads();
+  }
   const float total = D.total;
   if (tid == 0) a.wtot[2 * row] = total;
   path = kWideTotal;

@@ -1,9 +1,10 @@
 """GPU parity of the draws over a row's whole distribution (top-p without
 top-k, min-p alone, temperature only, top-k above 1024) against the oracle:
 tokens equal, at the edges of the tiles (1024 logits), of the pieces sorted at
-a time (4096 weights) and of the tile limit (262,144 logits), over one launch
-or two, 16-byte aligned rows and others, and over weights that all differ,
-come in long runs, or are all equal."""
+a time (4096 weights) and of a row's 256 tiles (262,144 logits: beyond, one
+workgroup's tiles are longer and the wide pass chains them 256 at a time),
+over one launch or two, 16-byte aligned rows and others, and over weights that
+all differ, come in long runs, or are all equal."""
 import numpy as np
 import pytest
 
@@ -132,3 +133,44 @@ def test_one_launch_grids(hip, oracle, B, V):
         want = oracle.sample_rows(x, p, u)["tokens"]
         bad = np.flatnonzero(got != want)
         assert bad.size == 0, (bad, got[bad], want[bad])
+
+
+GRID = [(9, 262143), (9, 262144), (9, 262145), (12, 262208), (2, 1048577), (40, 70001), (64, 50257), (128, 50257)]
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("B,V", GRID)
+def test_finish_grid(hip, oracle, B, V, bf16):
+    """Two launches (more than 512 workgroups of 4096 logits): nucleus and
+    min-p rows through the wide pass, which the path codes show, and
+    temperature-only rows split over workgroups, in units of one chunk (up to
+    768 workgroups) and of four, on both sides of 256 tiles and 256 chunks,
+    rows of any alignment, with and without logprobs."""
+    import torch
+    from hi_amd import sampler as S
+    n = B * ((V + 4095) // 4096)
+    assert n > 512 and B * ((V + 16383) // 16384) < 1024
+    x = _rows("spiked", B, V, V + B)
+    p = _params(B)
+    p["top_k"][4::5] = 40
+    u = np.random.default_rng(V).random(B).astype(F32)
+    logits = f32_to_bf16_bits(x) if bf16 else x
+    t = torch.from_numpy(logits.view(np.int16) if bf16 else logits).cuda()
+    t = t.view(torch.bfloat16) if bf16 else t
+    # (bf16 rows of top-p 0.999 list their whole distribution, whose distinct
+    # weights may pass the merge's table: finish_row then)
+    whole = np.flatnonzero((p["top_k"] == 0) & ((p["top_p"] < (0.99 if bf16 else 1)) | (p["min_p"] > 0)))
+    for n_lp in (0, 3):
+        smp = S.Sampler(B, V, n_lp)
+        print(f"finish grid B={B} V={V} bf16={bf16} logprobs={n_lp}", flush=True)
+        out = smp.sample(t, S.params_to_device(p), torch.from_numpy(u).cuda(), n_logprobs=n_lp)
+        torch.cuda.synchronize()
+        want = oracle.sample_rows(logits, p, u, n_logprobs=n_lp)
+        got = out["tokens"].cpu().numpy().view(np.uint32)
+        bad = np.flatnonzero(got != want["tokens"])
+        assert bad.size == 0, (bad, got[bad], want["tokens"][bad])
+        names = [S.WIDE_PATHS[int(c)] for c in S.debug_wide_paths(smp, B, V)[whole]]
+        assert names == ["wide"] * len(whole), names
+        if n_lp:
+            np.testing.assert_allclose(out["logprobs"].cpu().numpy(), want["logprobs"], rtol=1e-5, atol=0)
+            assert np.array_equal(out["logprob_ids"].cpu().numpy().view(np.uint32), want["logprob_ids"])
