@@ -160,6 +160,7 @@ void carve(hi_rocm::SampleArgs& a, void* ws, const hi_rocm::WorkspaceLayout& L) 
   a.done = (uint32_t*)(base + L.done);
   a.wstat = (hi_rocm::WideStat*)(base + L.wstat);
   a.wfold = (hi_rocm::ChunkFold*)(base + L.wfold);
+  a.wruns = (uint64_t*)(base + L.wruns);
   a.diag = (uint32_t*)(base + L.diag);
   a.wtot = (float*)(base + L.wtot);
   // Masked rows that do not start on 16 bytes stay with the general scan: the

@@ -93,13 +93,18 @@ struct WideStat {
 static_assert(sizeof(WideStat) == 136, "WideStat layout");
 
 // Per (row, chunk) result of the wide pass for a top-p row: the number of
-// weights it listed (those of the nucleus superset) and, per tile of 1024
-// logits, its map in the vocabulary-order fold for a start in its predicted
-// binade, and in the one below (DrawLds in sampler_draw.h holds a row's).
+// weights it listed (those of the nucleus superset), of the distinct values
+// it counted among them (f32 logits; kFoldNone: not counted) and, per tile of
+// 1024 logits, its map in the vocabulary-order fold for a start in its
+// predicted binade, and in the one below (DrawLds in sampler_draw.h holds a
+// row's).
 constexpr int kChunkTiles = 16;  // tiles of the largest chunk
+constexpr int kChunkRuns = 512;  // distinct values kept per chunk
+constexpr uint32_t kFoldNone = 0xffffffffu;  // n: the chunk's table overflowed
 struct ChunkFold {
   uint32_t n;
-  uint32_t pad[3];
+  uint32_t nr;
+  uint32_t pad[2];
   fold::Map map[kChunkTiles], low[kChunkTiles];
   uint32_t bin[kChunkTiles];
 };
@@ -136,6 +141,7 @@ struct SampleArgs {
   uint32_t* done;      // [kDoneRows] chunks of the row finished (zero between launches)
   WideStat* wstat;     // [B][n_chunks]
   ChunkFold* wfold;    // [B][n_chunks]
+  uint64_t* wruns;     // [B][n_chunks][kChunkRuns]: the distinct values of a chunk's listed weights
   uint32_t* diag;      // [B] how the wide pass finished each top-p row (WidePath)
   float* wtot;         // [B][2] the wide pass's normaliser and candidate total (debug export)
 };
@@ -145,9 +151,11 @@ struct SampleArgs {
 enum WidePath : uint32_t {
   kWideDone = 1,          // finished by the wide pass
   kWideNoStats = 2,       // a chunk's statistics were not written by this call's pass, or no finite logit
+  kWideChunkFull = 3,     // a unit's table of distinct weights overflowed
   kWideTotal = 4,         // the normaliser is not positive and finite (argmax fallback)
+  kWideMergeFull = 5,     // the row's table of distinct weights overflowed
   kWideNoCutoff = 6,      // the cutoff lies outside the superset
-  kWideDrawFail = 7,      // the candidate total is not positive and finite
+  kWideDrawFail = 7,      // the candidate total is not positive and finite, or the drawn index was not found
   // rows of the row kernel
   kRowPathMinp = 8,       // the min-p support finish
   kRowPathLists = 9,      // the candidate lists' finish (finish_core)
@@ -163,7 +171,7 @@ constexpr int kFusedMaxRows = kFusedMaxWorkgroups;
 constexpr int kDoneRows = 65536;
 
 struct WorkspaceLayout {
-  size_t stats, cand, ws_s, ws_w, ws_list, done, wstat, wfold, diag, wtot, total;
+  size_t stats, cand, ws_s, ws_w, ws_list, done, wstat, wfold, wruns, diag, wtot, total;
   int64_t slots;       // (row, chunk) records reserved
   int64_t list_stride;
 };
@@ -189,6 +197,7 @@ inline WorkspaceLayout workspace_layout_slots(int max_batch, int V, int64_t slot
   L.stats = off; off = align(off + (size_t)L.slots * sizeof(ChunkStat));
   L.wstat = off; off = align(off + (size_t)L.slots * sizeof(WideStat));
   L.wfold = off; off = align(off + (size_t)L.slots * sizeof(ChunkFold));
+  L.wruns = off; off = align(off + (size_t)L.slots * kChunkRuns * sizeof(uint64_t));
   L.diag = off; off = align(off + (size_t)max_batch * sizeof(uint32_t));
   L.wtot = off; off = align(off + (size_t)max_batch * 2 * sizeof(float));
   L.cand = off; off = align(off + (size_t)L.slots * kFast * sizeof(uint64_t));

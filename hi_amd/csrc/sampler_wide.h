@@ -22,11 +22,14 @@ namespace hi_rocm {
 //      for the binade its predicted start lies in (sampler_draw.h);
 //   3. lists its weights >= w_lo with their indexes (bf16 logits: their
 //      distinct values with counts, an LDS hash: thousands of logits share
-//      one weight);
+//      one weight); f32 weights that turn out to share values in a sample
+//      are counted by value as well (f32 logits that hold bf16 values, or
+//      few levels);
 //   4. bumps the row's counter; the last workgroup finishes the row: wave 0
 //      chains the tile maps into the exact normaliser while the others
 //      gather the lists, then the ranks are sorted and folded (draw_ranks;
-//      bf16: runs of equal weights in closed form, wide_finish_runs).
+//      bf16, and long f32 lists of few values: runs of equal weights in
+//      closed form, wide_finish_runs).
 // A temperature-only row's workgroups sum its 256 reference chunks instead,
 // one wave a chunk, and the last one draws.
 // Rows whose chunks took the select pass's exact path, whose nucleus is not
@@ -48,11 +51,10 @@ namespace hi_rocm {
 constexpr float kWideMargin = 0.005f;  // extra probability mass of the superset
 constexpr int kWideGBins = 64;         // threshold bins (binades of w below M)
 constexpr int kWideTile = 64 * kDrawPer;
-constexpr int kWideHash = 2048;        // distinct superset weights of a chunk, and of a row (bf16 logits)
+constexpr int kWideHash = 2048;        // distinct superset weights of a chunk, and of a row
 constexpr int kWideLog2 = 11;
 static_assert((1 << kWideLog2) == kWideHash, "hash size");
 constexpr int kWideProbes = 64;
-constexpr uint32_t kFoldNone = 0xffffffffu;  // ChunkFold.n: the chunk's table overflowed
 constexpr int kWidePre = kSelChunkLarge / kWideTile / (NT / 64);  // tiles of a wave, at most
 static_assert(kSelChunkLarge / kWideTile == kChunkTiles, "a chunk's tile records");
 
@@ -78,12 +80,12 @@ struct WideChunkLds {
   float w_lo;
   float tsum[kChunkTiles];
   uint32_t wcnt[NT / 64];
-  uint32_t n, last;
-  // bf16 rows: the superset's distinct weights
+  uint32_t n, nr, last;
+  // the superset's distinct weights
   uint32_t hkey[kWideHash], hcnt[kWideHash], hmin[kWideHash];
 };
 
-// LDS of the row finish over runs of equal weights (bf16 logits).
+// LDS of the row finish over runs of equal weights.
 struct WideRunLds {
   fold::WgLds<NT> fl;
   union {
@@ -104,6 +106,7 @@ struct WideRunLds {
   uint8_t pe[kWideHash + 4];
   uint32_t noff[kDrawChunks + 1];
   uint32_t cntc[kDrawChunks];  // the drawn weight's multiplicity per chunk
+  uint8_t listed[kDrawChunks];  // the unit's entries are its list (else runs)
   uint32_t cnt, rsel, csel, tok;
 };
 
@@ -115,7 +118,7 @@ __device__ __forceinline__ uint32_t wide_hash(uint32_t key, int log2n) {
 // into an LDS table of 2^log2n slots (key 0 = empty; weights here are > 0).
 // Returns false when kWideProbes slots in a row hold other weights (a table
 // that fills up would otherwise be searched end to end for every weight); a
-// thread inserts nothing more then.
+// thread soon inserts nothing more then.
 __device__ __forceinline__ bool wide_insert(uint32_t* hkey, uint32_t* hcnt, uint32_t* hmin, int log2n,
                                             uint32_t key, uint32_t count, uint32_t idx) {
   const uint32_t mask = (1u << log2n) - 1u;
@@ -297,6 +300,64 @@ __device__ __forceinline__ float wide_row_max(const SampleArgs& a, int row, cons
   return finitef_(ml) ? ml / cfg.t_eff : -__builtin_inff();
 }
 
+// Counts the n listed weights of a unit by value into its wruns, when a
+// sample of them shares values; returns the number of values, or kFoldNone.
+// For lists that a row could not sort at once (kDrawPiece, by the unit's
+// share): there the ranks take a sort and two folds a piece, and none of
+// that when a value repeats more often than a piece is long.  64 f32 rows of
+// 151,936, nucleus: bf16 values 416 -> 156 us, seven levels 3,960 -> 203, all
+// equal 25 ms -> 335 us; values that all differ 413 -> 416 (the sample).
+__device__ __forceinline__ uint32_t wide_count_runs(WideChunkLds& L, const SampleArgs& a, int row, const WideUnits& wu,
+                                                    int unit, const uint64_t* list, uint32_t n) {
+  const int tid = threadIdx.x;
+  const uint32_t c0 = (uint32_t)(unit * wu.len);
+  for (int h = tid; h < kWideHash; h += NT) { L.hkey[h] = 0u; L.hcnt[h] = 0u; L.hmin[h] = 0xffffffffu; }
+  if (tid == 0) L.nr = 0u;
+  __syncthreads();
+  // the sample: up to NT weights spread over the list (keys without counts)
+  const uint32_t ns = min(n, (uint32_t)NT);
+  if ((uint32_t)tid < ns) {
+    const uint64_t e = list[(uint32_t)tid * (n / ns)];
+    (void)wide_insert(L.hkey, L.hcnt, L.hmin, kWideLog2, (uint32_t)(e >> 32), 0u, (uint32_t)e - c0);
+  }
+  __syncthreads();
+  uint32_t mine = 0u;
+  for (int h = tid; h < kWideHash; h += NT) mine += L.hkey[h] != 0u ? 1u : 0u;
+  mine = wave_sum_u32(mine);
+  if ((tid & 63) == 0) atomicAdd(&L.nr, mine);
+  __syncthreads();
+  const bool few = L.nr <= ns * 3u / 4u;
+  __syncthreads();
+  if (!few) return kFoldNone;
+  if (tid == 0) L.nr = 0u;
+  bool full = false;
+  constexpr int kU = 8;
+  for (uint32_t base = 0; base < n; base += kU * NT) {
+    uint64_t e[kU];
+    #pragma unroll
+    for (int k = 0; k < kU; ++k) {
+      const uint32_t p = base + (uint32_t)(k * NT + tid);
+      e[k] = p < n ? list[p] : 0ull;
+    }
+    #pragma unroll
+    for (int k = 0; k < kU; ++k)
+      if (e[k] != 0ull && !full)
+        full = !wide_insert(L.hkey, L.hcnt, L.hmin, kWideLog2, (uint32_t)(e[k] >> 32), 1u, (uint32_t)e[k] - c0);
+  }
+  if (__syncthreads_or(full)) return kFoldNone;
+  // (the row's last unit may have fewer chunks)
+  const uint32_t cap = (uint32_t)(kChunkRuns * min(wu.chunks, a.n_chunks - unit * wu.chunks));
+  uint64_t* out = a.wruns + ((int64_t)row * a.n_chunks + (int64_t)unit * wu.chunks) * kChunkRuns;
+  for (int h = tid; h < kWideHash; h += NT) {
+    const uint32_t k = L.hkey[h];
+    if (k == 0u) continue;
+    const uint32_t p = atomicAdd(&L.nr, 1u);
+    if (p < cap) out[p] = ((uint64_t)k << 32) | ((uint64_t)L.hcnt[h] << 16) | (uint64_t)L.hmin[h];
+  }
+  __syncthreads();
+  return L.nr <= cap ? L.nr : kFoldNone;
+}
+
 // Steps 2-3 for one (unit, row), with the row's M and w_lo and the unit's
 // predicted start S.
 __device__ __forceinline__ void wide_chunk_work(WideChunkLds& L, const SampleArgs& a, int row, const WideUnits& wu,
@@ -348,9 +409,9 @@ __device__ __forceinline__ void wide_chunk_work(WideChunkLds& L, const SampleArg
     for (int q = 0; q < kDrawPer; ++q) mk |= x[i][q] > 0.f && x[i][q] >= w_lo ? 1u << q : 0u;
     if (__ballot(mk != 0u) == 0ull) continue;
     if (runs) {
-      for (; mk != 0u && !full; mk &= mk - 1u) {
+      for (mk = full ? 0u : mk; mk != 0u; mk &= mk - 1u) {
         const int q = __ffs((int)mk) - 1;
-        full = !wide_insert(L.hkey, L.hcnt, L.hmin, kWideLog2, __float_as_uint(tr[lane * kTrLd + q]), 1u,
+        full |= !wide_insert(L.hkey, L.hcnt, L.hmin, kWideLog2, __float_as_uint(tr[lane * kTrLd + q]), 1u,
                              (uint32_t)(t0 - c0 + lane * kDrawPer + q));
       }
       continue;
@@ -373,7 +434,14 @@ __device__ __forceinline__ void wide_chunk_work(WideChunkLds& L, const SampleArg
     }
     __syncthreads();
   }
-  if (tid == 0) cf->n = ovf ? kFoldNone : L.n;
+  const uint32_t n = L.n;
+  uint32_t nr = kFoldNone;
+  if (__builtin_expect(!runs && n >= 64u && n * (uint32_t)wu.n > (uint32_t)kDrawPiece, 0))
+    nr = wide_count_runs(L, a, row, wu, unit, list, n);
+  if (tid == 0) {
+    cf->n = ovf ? kFoldNone : n;
+    cf->nr = nr;
+  }
   #pragma unroll
   for (int i = 0; i < kWidePre; ++i) {
     const int tl = i * (NT / 64) + wid;
@@ -494,14 +562,18 @@ struct WideListSrc {
   }
 };
 
-// Calls f(c, e) for every run entry e of chunk c of `row`, in parallel (the
-// chunks' offsets in F.noff, n_all entries).
-template <typename Fn>
+// Calls f(unit, weight bits, count, index) for every entry of the row's
+// units, in parallel (the units' offsets in F.noff, n_all entries): a value
+// with its count and smallest index, or a listed weight (F.listed) with its
+// own.
+template <bool BF16, typename Fn>
 __device__ __forceinline__ void wide_for_each_run(WideRunLds& F, const SampleArgs& a, int row, const WideUnits& wu,
                                                   int n_all, Fn f) {
   constexpr int kU = 8;
   const int tid = threadIdx.x;
   const uint64_t* list = a.ws_list + (int64_t)row * a.list_stride;
+  const uint64_t* runs = BF16 ? list : a.wruns + (int64_t)row * a.n_chunks * kChunkRuns;
+  const int stride = BF16 ? wu.len : wu.chunks * kChunkRuns;
   for (int base = 0; base < n_all; base += kU * NT) {
     uint64_t v[kU];
     int c[kU];
@@ -512,28 +584,42 @@ __device__ __forceinline__ void wide_for_each_run(WideRunLds& F, const SampleArg
       #pragma unroll
       for (int k = 0; k < kU; ++k) c[k] = (int)F.noff[c[k] + st] <= base + k * NT + tid ? c[k] + st : c[k];
     }
-    #pragma unroll
-    for (int k = 0; k < kU; ++k) {
-      const int p = base + k * NT + tid;
-      v[k] = p < n_all ? list[(int64_t)c[k] * wu.len + (p - (int)F.noff[c[k]])] : 0ull;
+    uint32_t one = 0u;  // bit k: a listed weight
+    if (!BF16) {
+      #pragma unroll
+      for (int k = 0; k < kU; ++k) one |= F.listed[c[k]] != 0 ? 1u << k : 0u;
     }
     #pragma unroll
-    for (int k = 0; k < kU; ++k)
-      if (base + k * NT + tid < n_all) f(c[k], v[k]);
+    for (int k = 0; k < kU; ++k) {
+      const int p = base + k * NT + tid, at = p - (int)F.noff[c[k]];
+      const uint64_t* from = (one >> k) & 1u ? list + (int64_t)c[k] * wu.len : runs + (int64_t)c[k] * stride;
+      v[k] = p < n_all ? from[at] : 0ull;
+    }
+    #pragma unroll
+    for (int k = 0; k < kU; ++k) {
+      if (base + k * NT + tid >= n_all) continue;
+      const uint32_t e = (uint32_t)v[k];
+      const bool w = (one >> k) & 1u;
+      f(c[k], (uint32_t)(v[k] >> 32), w ? 1u : e >> 16, w ? e : (uint32_t)(c[k] * wu.len) + (e & 0xffffu));
+    }
   }
   __syncthreads();
 }
 
-// The ranks of a bf16 row, whose superset has few distinct weights: the
-// chunks' runs merged by weight and sorted, the rank-order folds over runs
-// of equal weights in closed form.  `mine`: this thread's chunk's runs,
-// n_all their sum; returns the token or 0xffffffff.  All threads call it.
+// The ranks of a row whose superset has few distinct weights: the units'
+// runs merged by weight and sorted, the rank-order folds over runs of equal
+// weights in closed form.  `mine`: the entries of unit threadIdx.x, `listed`:
+// they are its list; returns the token, or 0xffffffff (path kWideMergeFull:
+// the table of distinct weights overflowed).  All threads call it.
+template <bool BF16>
 __device__ __forceinline__ uint32_t wide_finish_runs(WideRunLds& F, const SampleArgs& a, int row, const RowCfg& cfg,
-                                                     const WideUnits& wu, float w_lo, float total, uint32_t mine, uint32_t& path) {
+                                                     const WideUnits& wu, float w_lo, float total, uint32_t mine, bool listed,
+                                                     uint32_t& path) {
   const int tid = threadIdx.x;
   const int nch = wu.n;
   uint32_t n_all;
   F.noff[tid] = block_excl_scan_u32<NT>(mine, F.fl.wcnt, &n_all);
+  F.listed[tid] = listed ? 1u : 0u;
   if (tid == 0) F.noff[NT] = n_all;
 
   // c. merge the chunks' runs by weight
@@ -545,12 +631,10 @@ __device__ __forceinline__ uint32_t wide_finish_runs(WideRunLds& F, const Sample
   if (tid == 0) F.cnt = 0u;
   __syncthreads();
   bool full = false;
-  auto insert = [&](int c, uint64_t e) {
-    if (!full) full = !wide_insert(F.u.mg.hkey, F.u.mg.hcnt, F.u.mg.hmin, kWideLog2, (uint32_t)(e >> 32),
-                                   (uint32_t)(e >> 16) & 0xffffu, (uint32_t)(c * wu.len) + ((uint32_t)e & 0xffffu));
-  };
-  wide_for_each_run(F, a, row, wu, (int)n_all, insert);
-  path = kWideNoCutoff;
+  wide_for_each_run<BF16>(F, a, row, wu, (int)n_all, [&](int, uint32_t key, uint32_t count, uint32_t idx) {
+    if (!full) full = !wide_insert(F.u.mg.hkey, F.u.mg.hcnt, F.u.mg.hmin, kWideLog2, key, count, idx);
+  });
+  path = kWideMergeFull;
   if (__syncthreads_or(full)) return 0xffffffffu;
   path = kWideDrawFail;
   // d. distinct weights, descending: the table's used slots compacted in
@@ -682,8 +766,8 @@ __device__ __forceinline__ uint32_t wide_finish_runs(WideRunLds& F, const Sample
   __syncthreads();
   F.cntc[tid] = 0u;
   __syncthreads();
-  wide_for_each_run(F, a, row, wu, (int)n_all, [&](int c, uint64_t e) {
-    if ((uint32_t)(e >> 32) == key) F.cntc[c] = (uint32_t)(e >> 16) & 0xffffu;
+  wide_for_each_run<BF16>(F, a, row, wu, (int)n_all, [&](int c, uint32_t k, uint32_t count, uint32_t) {
+    if (k == key) atomicAdd(&F.cntc[c], count);
   });
   if (tid < 64) {
     // the chunk holding the cp-th match: an inclusive scan of the chunks'
@@ -782,21 +866,41 @@ __device__ __forceinline__ uint32_t wide_finish(DrawLds<NT>& D, const SampleArgs
     }
   };
   load_tiles(0);
-  for (int b = tid; b < kDrawBins + kDrawBins / 32; b += NT) D.hist[b] = 0u;
   uint32_t n_all;
-  D.noff[tid] = block_excl_scan_u32<NT>(mine, D.red, &n_all);
-  if (tid == 0) {
-    D.noff[NT] = n_all;
-    D.n = n_all;
-  }
+  auto lists = [&]() {
+    for (int b = tid; b < kDrawBins + kDrawBins / 32; b += NT) D.hist[b] = 0u;
+    D.noff[tid] = block_excl_scan_u32<NT>(mine, D.red, &n_all);
+    if (tid == 0) {
+      D.noff[NT] = n_all;
+      D.n = n_all;
+    }
+  };
+  lists();
   static_assert(NT == kDrawChunks && NT == kDrawTiles, "a thread per chunk and per tile");
   __syncthreads();
   const WideListSrc src{wu, r, a.ws_list + (int64_t)row * a.list_stride, (int)n_all, !(w_lo > cfg.min_p)};
   const bool one = n_all <= (uint32_t)kDrawPiece;  // every listed weight fits a piece
+  // f32: the units' values, where counted, when they halve the entries
+  bool counted = false;
+  uint32_t entries = mine;
+  bool listed = true;
+  if (!runs && !one) {
+    const uint32_t nr = tid < nch ? folds[tid].nr : kFoldNone;
+    listed = nr == kFoldNone;
+    entries = listed ? mine : nr;
+    uint32_t n_runs;
+    block_excl_scan_u32<NT>(entries, D.red, &n_runs);
+    counted = n_runs <= n_all / 2u;
+  }
   constexpr uint32_t kTop = (uint32_t)((kDrawAll - 1u) >> 23);
+  auto histogram = [&](int p0, int stride) {
+    src.each(D, p0, stride, [&](int, uint64_t e) {
+      atomicAdd(&D.hist[draw_slot(draw_bin(__uint_as_float((uint32_t)(e >> 32))))], 1u);
+    });
+  };
   if (wid == 0) {
     draw_chain<NT>(D, r, 0, min(nt, kDrawTiles), -0.0f);
-  } else if (runs) {
+  } else if (runs || counted) {
   } else if (one) {
     int p = tid - 64;  // entries in order: p, p + 192, ...
     src.each(D, tid - 64, NT - 64, [&](int, uint64_t e) {
@@ -804,9 +908,7 @@ __device__ __forceinline__ uint32_t wide_finish(DrawLds<NT>& D, const SampleArgs
       p += NT - 64;
     });
   } else {
-    src.each(D, tid - 64, NT - 64, [&](int, uint64_t e) {
-      atomicAdd(&D.hist[draw_slot(draw_bin(__uint_as_float((uint32_t)(e >> 32))))], 1u);
-    });
+    histogram(tid - 64, NT - 64);
   }
   __syncthreads();
   for (int t0 = kDrawTiles; t0 < nt; t0 += kDrawTiles) {
@@ -819,11 +921,25 @@ __device__ __forceinline__ uint32_t wide_finish(DrawLds<NT>& D, const SampleArgs
   if (tid == 0) a.wtot[2 * row] = total;
   path = kWideTotal;
   if (!(total > 0.f) || !finitef_(total)) return 0xffffffffu;  // argmax_host fallback (finish_row)
-  path = kWideNoCutoff;
+  path = kWideChunkFull;
   if (ovf) return 0xffffffffu;
+  path = kWideNoCutoff;
   if (runs) {
     __syncthreads();
-    return wide_finish_runs(reinterpret_cast<WideRunLds&>(D), a, row, cfg, wu, w_lo, total, mine, path);
+    return wide_finish_runs<true>(reinterpret_cast<WideRunLds&>(D), a, row, cfg, wu, w_lo, total, mine, false, path);
+  }
+  if (__builtin_expect(counted, 0)) {
+    __syncthreads();
+    const uint32_t tok = wide_finish_runs<false>(reinterpret_cast<WideRunLds&>(D), a, row, cfg, wu, w_lo, total, entries,
+                                                 listed, path);
+    if (tok != 0xffffffffu || path != kWideMergeFull) return tok;
+    // too many values after all: the ranks from the lists
+    __syncthreads();
+    lists();
+    __syncthreads();
+    histogram(tid, NT);
+    __syncthreads();
+    path = kWideNoCutoff;
   }
   uint64_t lo = (uint64_t)max(__float_as_uint(w_lo), 1u) << 23;
   uint32_t bin = (uint32_t)kDrawBins;

@@ -174,3 +174,42 @@ def test_finish_grid(hip, oracle, B, V, bf16):
         if n_lp:
             np.testing.assert_allclose(out["logprobs"].cpu().numpy(), want["logprobs"], rtol=1e-5, atol=0)
             assert np.array_equal(out["logprob_ids"].cpu().numpy().view(np.uint32), want["logprob_ids"])
+
+
+@pytest.mark.parametrize("kind", ["levels", "equal", "bf16 values", "both", "own levels", "flat"])
+@pytest.mark.parametrize("B,V", [(16, 151936), (56, 70003)])
+def test_f32_rows_of_few_values(hip, oracle, B, V, kind):
+    """f32 rows whose long lists share values: counted by value in units of
+    one chunk and of four; rows with a unit of other values, which stays
+    listed beside counted ones; units with levels of their own, too many together for the merge's table
+    (their ranks come from the lists after all); rows that share none."""
+    import torch
+    from hi_amd import sampler as S
+    assert B * ((V + 4095) // 4096) > 512
+    rng = np.random.default_rng(V)
+    x = rng.normal(0, 1.5, (B, V))
+    if kind == "levels":
+        x = np.round(x)
+    elif kind == "equal":
+        x = np.full((B, V), 0.25)
+    elif kind == "both":
+        x[:, :-1000] = np.round(x[:, :-1000] * 4) / 4
+    elif kind == "own levels":
+        x = np.round(x * 64) / 64 + np.arange(V) // 4096 * 2.0 ** -12
+    x = x.astype(F32)
+    if kind == "bf16 values":
+        x = (f32_to_bf16_bits(x).astype(np.uint32) << 16).view(F32)
+    p = _params(B)
+    p["top_k"][4::5] = 0
+    u = rng.random(B).astype(F32)
+    smp = S.Sampler(B, V)
+    print(f"few values B={B} V={V} {kind}", flush=True)
+    out = smp.sample(torch.from_numpy(x).cuda(), S.params_to_device(p), torch.from_numpy(u).cuda())
+    torch.cuda.synchronize()
+    want = oracle.sample_rows(x, p, u)["tokens"]
+    got = out["tokens"].cpu().numpy().view(np.uint32)
+    bad = np.flatnonzero(got != want)
+    assert bad.size == 0, (bad, got[bad], want[bad])
+    nucleus = np.flatnonzero(p["top_p"] < 0.99)
+    names = [S.WIDE_PATHS[int(c)] for c in S.debug_wide_paths(smp, B, V)[nucleus]]
+    assert names == ["wide"] * len(nucleus), names
