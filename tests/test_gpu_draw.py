@@ -213,3 +213,39 @@ def test_f32_rows_of_few_values(hip, oracle, B, V, kind):
     nucleus = np.flatnonzero(p["top_p"] < 0.99)
     names = [S.WIDE_PATHS[int(c)] for c in S.debug_wide_paths(smp, B, V)[nucleus]]
     assert names == ["wide"] * len(nucleus), names
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("B,V,n_hist", [(3, 50257, 3500), (45, 50257, 3500), (5, 50304, 700), (4, 16387, 16000)])
+def test_dense_histories(hip, oracle, B, V, n_hist, bf16):
+    """Greedy and top-k rows whose histories mark more than 64 tokens of a
+    chunk (the select pass leaves them out of its maxima), the likeliest
+    tokens among them, with penalties that keep, lower or raise them, one
+    launch and two, with logprobs."""
+    import torch
+    from hi_amd import sampler as S
+    rng = np.random.default_rng(V + B)
+    x = _rows("spiked", B, V, V + B)
+    logits = f32_to_bf16_bits(x) if bf16 else x
+    p = np.zeros(B, ROW_PARAMS_DTYPE)
+    p["temperature"] = np.where(np.arange(B) % 3 == 0, 0.0, 0.9)
+    p["top_k"], p["top_p"] = 40, 0.95
+    p["repetition_penalty"] = np.array([1.3, 1.0, 0.8], F32)[np.arange(B) % 3]
+    p["frequency_penalty"] = np.array([0.0, 0.2, -0.1], F32)[np.arange(B) % 3]
+    ids = np.stack([np.concatenate([np.argsort(x[b])[-30:], rng.permutation(V)[:n_hist]]) for b in range(B)])
+    off = (np.arange(B + 1) * ids.shape[1]).astype(np.uint32)
+    ids = ids.astype(np.uint32).ravel()
+    cnt = rng.integers(1, 4, ids.size).astype(np.uint32)
+    u = rng.random(B).astype(F32)
+    t = torch.from_numpy(logits.view(np.int16) if bf16 else logits).cuda()
+    i32 = lambda a: torch.from_numpy(a.view(np.int32)).cuda()  # noqa: E731
+    print(f"dense histories B={B} V={V} bf16={bf16}", flush=True)
+    out = S.Sampler(B, V, 5).sample(t.view(torch.bfloat16) if bf16 else t, S.params_to_device(p),
+                                    torch.from_numpy(u).cuda(), i32(off), i32(ids), i32(cnt), n_logprobs=5)
+    torch.cuda.synchronize()
+    want = oracle.sample_rows(logits, p, u, off, ids, cnt, n_logprobs=5)
+    got = out["tokens"].cpu().numpy().view(np.uint32)
+    bad = np.flatnonzero(got != want["tokens"])
+    assert bad.size == 0, (bad, got[bad], want["tokens"][bad])
+    np.testing.assert_allclose(out["logprobs"].cpu().numpy(), want["logprobs"], rtol=1e-5, atol=1e-6)
+    assert np.array_equal(out["logprob_ids"].cpu().numpy().view(np.uint32), want["logprob_ids"])
