@@ -156,6 +156,7 @@ enum WidePath : uint32_t {
   kWideMergeFull = 5,     // the row's table of distinct weights overflowed
   kWideNoCutoff = 6,      // the cutoff lies outside the superset
   kWideDrawFail = 7,      // the candidate total is not positive and finite, or the drawn index was not found
+  kWideLongList = 11,     // too long a list of distinct weights
   // rows of the row kernel
   kRowPathMinp = 8,       // the min-p support finish
   kRowPathLists = 9,      // the candidate lists' finish (finish_core)

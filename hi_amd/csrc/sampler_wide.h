@@ -55,6 +55,10 @@ constexpr int kWideHash = 2048;        // distinct superset weights of a chunk, 
 constexpr int kWideLog2 = 11;
 static_assert((1 << kWideLog2) == kWideHash, "hash size");
 constexpr int kWideProbes = 64;
+// A row of distinct weights whose list exceeds V / kWideListShare takes
+// finish_row: 64 f32 nucleus rows of 151,936, about everything listed 8,830 us
+// by the list and 2,831 by the row, about a seventh 418 and 537.
+constexpr int kWideListShare = 4;
 constexpr int kWidePre = kSelChunkLarge / kWideTile / (NT / 64);  // tiles of a wave, at most
 static_assert(kSelChunkLarge / kWideTile == kChunkTiles, "a chunk's tile records");
 
@@ -884,7 +888,7 @@ __device__ __forceinline__ uint32_t wide_finish(DrawLds<NT>& D, const SampleArgs
   bool counted = false;
   uint32_t entries = mine;
   bool listed = true;
-  if (!runs && !one) {
+  if (__builtin_expect(!runs && !one, 0)) {
     const uint32_t nr = tid < nch ? folds[tid].nr : kFoldNone;
     listed = nr == kFoldNone;
     entries = listed ? mine : nr;
@@ -892,6 +896,11 @@ __device__ __forceinline__ uint32_t wide_finish(DrawLds<NT>& D, const SampleArgs
     block_excl_scan_u32<NT>(entries, D.red, &n_runs);
     counted = n_runs <= n_all / 2u;
   }
+  // A piece of a long list costs more than one from the row's weights, which
+  // stream without a search for each entry's unit.
+  const bool too_long = n_all > (uint32_t)(a.V / kWideListShare);
+  path = kWideLongList;
+  if (__builtin_expect(!runs && !counted && too_long, 0)) return 0xffffffffu;
   constexpr uint32_t kTop = (uint32_t)((kDrawAll - 1u) >> 23);
   auto histogram = [&](int p0, int stride) {
     src.each(D, p0, stride, [&](int, uint64_t e) {
@@ -934,6 +943,7 @@ __device__ __forceinline__ uint32_t wide_finish(DrawLds<NT>& D, const SampleArgs
                                                  listed, path);
     if (tok != 0xffffffffu || path != kWideMergeFull) return tok;
     // too many values after all: the ranks from the lists
+    if (too_long) return tok;
     __syncthreads();
     lists();
     __syncthreads();
