@@ -221,7 +221,7 @@ hipError_t launch_sample(const SampleArgs& a, hipStream_t stream, const LaunchEv
   e = launch_select(a, stream);
   if (e == hipSuccess) e = record(le, 1, stream);
   if (e != hipSuccess) return e;
-  const WideUnits wu = wide_units(a.B, a.V, a.chunk, a.n_chunks);
+  const WideUnits wu = wide_units(a.chunk, a.n_chunks);
   const int64_t n_wg = (int64_t)(1 + ((wu.n - 1) | 1)) * a.B;
   if (n_wg * NT >= ((int64_t)1 << 32)) return hipErrorInvalidConfiguration;  // 1-D grid of work-items
   const size_t lds = finish_grid_lds();

@@ -30,14 +30,14 @@ namespace hi_rocm {
 //      gather the lists, then the ranks are sorted and folded (draw_ranks;
 //      bf16, and long f32 lists of few values: runs of equal weights in
 //      closed form, wide_finish_runs).
-// A temperature-only row's workgroups sum its 256 reference chunks instead,
-// one wave a chunk, and the last one draws.
+// A temperature-only row's workgroups sum its 256 reference chunks instead, a
+// quad of lanes a chunk, and the last one draws.
 // Rows whose chunks took the select pass's exact path, whose nucleus is not
 // inside the listed weights, or of more than 256 units take finish_row.
 //
 // A workgroup takes a unit of one or several select chunks (WideUnits): every
-// workgroup of a row repeats the row statistics (about 5 us), so once the
-// grid fills the chip a few times, fewer and larger units win.
+// workgroup of a row repeats the row statistics (about 5 us), so fewer and
+// larger units win.
 //
 // Measured against the form before it (a workgroup's weights and maps held
 // in LDS with crossing records, distinct weights in LDS hash tables, runs
@@ -68,10 +68,12 @@ struct WideUnits {
   int len;     // logits of one
   int chunks;  // select chunks of one
 };
-__host__ __device__ inline WideUnits wide_units(int B, int V, int chunk, int n_chunks) {
-  // 64 nucleus rows of 151,936: 192 us with units of one chunk, 122 us
-  // with units of four; 32 masked rows: 107 and 86 us
-  const int g = chunk < kSelChunkLarge && ((int64_t)B * n_chunks > 768 || n_chunks > kDrawChunks) ? kSelChunkLarge / chunk : 1;
+__host__ __device__ inline WideUnits wide_units(int chunk, int n_chunks) {
+  // units of kSelChunkLarge logits.  Units of one small chunk (one and four,
+  // nucleus): 14 f32 rows of 151,936 353 and 332 us, 26 rows 412 and 358; 20
+  // bf16 rows 116 and 99; 40 rows of 50,257 88 and 89, 56 rows 105 and 95,
+  // 80 rows 142 and 107 (smaller batches take one launch)
+  const int g = chunk < kSelChunkLarge ? kSelChunkLarge / chunk : 1;
   return WideUnits{(n_chunks + g - 1) / g, chunk * g, g};
 }
 
@@ -970,12 +972,14 @@ __device__ __forceinline__ uint32_t wide_finish(DrawLds<NT>& D, const SampleArgs
 // A temperature-only row's part of workgroup `chunk` < kTempSplit: the sums
 // of 64 of the 256 reference chunks, a quad each, to the row's ws_list.
 // Batches of up to kTempRows rows: beyond, one workgroup a row fills the chip
-// (256 rows of 151,936: 130 us, split 177 us).  (A
+// (bf16 rows of 151,936, one workgroup and split: 64 rows 64 and 59 us, 96
+// rows 68 and 69, 128 rows 81 and 95, 256 rows 124 and 176; of 50,257: 64 rows
+// 39 and 39, 128 rows 50 and 59).  (A
 // wave a chunk, folding 64 weights at a time, took 140 us for 64 rows of
 // 151,936 against 64 us for one workgroup a row: the folds are serial, so
 // they fill the chip only when every lane holds one.)
 constexpr int kTempSplit = 4;
-constexpr int kTempRows = 128;
+constexpr int kTempRows = 64;
 __device__ __forceinline__ void wide_temperature_work(WideChunkLds& L, const SampleArgs& a, int row, int chunk,
                                                       const DrawRow& r, float M) {
   const int tid = threadIdx.x;
