@@ -77,8 +77,6 @@ struct WgLds {
   Map tcarry[NTH];          // map of the thread's segment before its first run
   uint32_t tk[NTH];         // segment ordinal at the thread's first run
   Map seg_map[kWgSeg];      // map of segment k (its runs before boundary run k)
-  Map seg_alt[kWgSeg];      // the same terms in the binade below (fold_plan<.., true>)
-  Map walt[NTH / 64];
   uint32_t seg_A[kWgSeg];   // A at segment k's start (chain)
   uint32_t seg_e[kWgSeg];   // binade of segment k
   uint32_t bnd_run[kWgSeg]; // run index of boundary run k
@@ -121,18 +119,9 @@ __device__ __forceinline__ void block_of(int pos, int R, int& r0, int& r1) {
   r1 = r0 + J < R ? r0 + J : R;
 }
 
-// The map of a run in binade e, and (ALT) in the binade below.
-template <bool ALT>
-__device__ __forceinline__ void run_maps(float x, uint32_t m, int e, Map& mp, Map& ma) {
-  mp = run_map(classify(x, e), m);
-  if (ALT) ma = e > 1 ? run_map(classify(x, e - 1), m) : mp;
-}
-
 // Plan of runs [pos, R) from the predicted start value `base`.  pe has
-// room for R + 1 entries.  With ALT, every segment also gets its map in the
-// binade below its predicted one (seg_alt), for a start value that lags
-// the prediction.  Ends with a barrier.
-template <int NTH, typename TermF, typename MultF, bool ALT = false>
+// room for R + 1 entries.  Ends with a barrier.
+template <int NTH, typename TermF, typename MultF>
 __device__ __forceinline__ void fold_plan(WgLds<NTH>& L, uint8_t* pe, int pos, int R, double base, TermF term, MultF mult) {
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   int r0, r1;
@@ -188,22 +177,17 @@ __device__ __forceinline__ void fold_plan(WgLds<NTH>& L, uint8_t* pe, int pos, i
   //    (head) and after the last one (tail)
   uint32_t nbt = 0u;
   Map head = map_identity(), tail = map_identity();
-  Map head_a = map_identity(), tail_a = map_identity();
   for (int r = r0; r < r1; ++r) {
     const int e = pe[r];
     if (e != pe[r + 1]) {
       ++nbt;
       tail = map_identity();
-      tail_a = map_identity();
     } else {
-      Map mp, ma;
-      run_maps<ALT>(term(r), mult(r), e, mp, ma);
+      const Map mp = run_map(classify(term(r), e), mult(r));
       if (nbt) {
         tail = compose(tail, mp);
-        if (ALT) tail_a = compose(tail_a, ma);
       } else {
         head = compose(head, mp);
-        if (ALT) head_a = compose(head_a, ma);
       }
     }
   }
@@ -211,7 +195,6 @@ __device__ __forceinline__ void fold_plan(WgLds<NTH>& L, uint8_t* pe, int pos, i
   //    thread starts in, up to its first run; and the boundary ordinal
   uint32_t f = nbt ? 1u : 0u;
   Map m = nbt ? tail : head;
-  Map ma = nbt ? tail_a : head_a;
   uint32_t cnt = nbt;
   // (DPP steps: a lane with no lane below combines with zero flags, the
   // identity map and a zero count, which changes nothing)
@@ -221,10 +204,6 @@ __device__ __forceinline__ void fold_plan(WgLds<NTH>& L, uint8_t* pe, int pos, i
     const uint32_t of = dpp32<C, RM, BC>(0u, f);
     const Map om = dpp_map<C, RM, BC>(m);
     const uint32_t oc = dpp32<C, RM, BC>(0u, cnt);
-    if (ALT) {
-      const Map oa = dpp_map<C, RM, BC>(ma);
-      if (!f) ma = compose(oa, ma);
-    }
     seg_combine(of, om, f, m);
     cnt += oc;
   };
@@ -237,24 +216,20 @@ __device__ __forceinline__ void fold_plan(WgLds<NTH>& L, uint8_t* pe, int pos, i
   if (lane == 63) {
     L.wflag[wid] = f;
     L.wmap[wid] = m;
-    if (ALT) L.walt[wid] = ma;
     L.wcnt[wid] = cnt;
   }
   // exclusive: the inclusive value of the lane below (zero at lane 0)
   uint32_t ef = dpp32<0x138, 0xf, true>(0u, f);
   Map em = wave_map_prev(m);
-  Map ea = map_identity();
-  if (ALT) ea = wave_map_prev(ma);
   uint32_t ec = dpp32<0x138, 0xf, true>(0u, cnt);
   __syncthreads();
   uint32_t cf = 0u, cc = 0u, tot = 0u;
-  Map cm = map_identity(), ca = map_identity();
+  Map cm = map_identity();
   #pragma unroll
   for (int w = 0; w < NTH / 64; ++w) {
     if (w < wid) {
       uint32_t ff = L.wflag[w];
       Map mm = L.wmap[w];
-      if (ALT) ca = ff ? L.walt[w] : compose(ca, L.walt[w]);
       seg_combine(cf, cm, ff, mm);
       cf = ff;
       cm = mm;
@@ -262,7 +237,6 @@ __device__ __forceinline__ void fold_plan(WgLds<NTH>& L, uint8_t* pe, int pos, i
     }
     tot += L.wcnt[w];
   }
-  if (ALT && !ef) ea = compose(ca, ea);
   seg_combine(cf, cm, ef, em);  // previous waves, then the lanes below
   L.tcarry[tid] = em;
   L.tk[tid] = cc + ec;
@@ -271,27 +245,21 @@ __device__ __forceinline__ void fold_plan(WgLds<NTH>& L, uint8_t* pe, int pos, i
   //    (and the thread holding the last run, for the last segment)
   {
     uint32_t k = cc + ec;
-    Map cur = em, cura = ea;
+    Map cur = em;
     for (int r = r0; r < r1; ++r) {
       const int e = pe[r];
       if (e != pe[r + 1]) {
         L.seg_map[k] = cur;
-        if (ALT) L.seg_alt[k] = cura;
         L.seg_e[k] = (uint32_t)e;
         L.bnd_run[k] = (uint32_t)r;
         ++k;
         cur = map_identity();
-        cura = map_identity();
       } else {
-        Map mp, mq;
-        run_maps<ALT>(term(r), mult(r), e, mp, mq);
-        cur = compose(cur, mp);
-        if (ALT) cura = compose(cura, mq);
+        cur = compose(cur, run_map(classify(term(r), e), mult(r)));
       }
     }
     if (r0 < r1 && r1 == R) {
       L.seg_map[k] = cur;
-      if (ALT) L.seg_alt[k] = cura;
       L.seg_e[k] = pe[R];
     }
   }

@@ -20,8 +20,8 @@
 //                       workgroups finish the rows (spread over every XCD)
 //                       and whose other workgroups run the wide pass of
 //                       top-p and temperature-only rows.
-//   scan + finish       more than 256 logprobs, or rows not aligned for
-//                       vector loads: scan_generic_kernel, then
+//   scan + finish       more than 256 logprobs, or masked rows that do not
+//                       start on 16 bytes: scan_generic_kernel, then
 //                       finish_kernel, one workgroup per row.
 //
 // Per element: allowed-token mask, penalties from an LDS count table of the
@@ -603,11 +603,9 @@ struct Exp2TabLds {
 };
 
 struct FinLds {
-  uint64_t cbig[kGather];     // gathered candidates (32 KiB) -- also a fold tile
+  uint64_t cbig[kGather];     // gathered candidates (32 KiB)
   uint64_t buf[kBuf];         // selected candidates / rank keys
   uint32_t pay[kBuf];         // scaled-logit keys riding with buf
-  float fa[kBuf];             // weights in rank order
-  float fb[kBuf];             // w / total
   uint32_t hist[kBins];
   uint64_t mass[kBins];
   uint32_t aux[kBins];
@@ -618,7 +616,7 @@ struct FinLds {
   uint64_t red64b[NT / 64];
   uint32_t sel[4];
   uint32_t counter, n_ext, token, flag;
-  float fval0, fval1;
+  float fval1;
   uint64_t below;   // largest candidate left out of the selection
   uint32_t wmin;    // bits of the smallest selected weight
   uint64_t thr;     // the selection threshold of a one-wave select
@@ -627,8 +625,6 @@ struct FinLds {
   double lsum;      // finish_core_wave: log of the logprob normaliser
   uint64_t exptab[32];  // exact_expf's table (finish_lean and rank_candidates copy it)
 };
-constexpr int kTileFloats = kGather * 2;  // floats of the fold tile (cbig)
-
 
 // ==========================================================================
 // Finish phase (one workgroup per row)
@@ -736,13 +732,13 @@ __device__ __forceinline__ void sort_ranked(FinLds& fs, int n) {
   __syncthreads();
 }
 
-// Descending bitonic sort of the keys buf[0..n), n <= PER * NTH, keys only
-// (zero pads them and sorts last; equal keys are equal values), by NTH
-// threads.  PER consecutive elements per thread in registers: distances
-// below PER inside the thread, up to 32 * PER across the lanes of a wave
-// (DPP, swizzle and bpermute lane moves), 64 * PER and more through buf with
-// barriers.  buf has room for PER * NTH keys; all of them are written.
-template <int PER, int NTH = NT>
+// Descending bitonic sort of the keys buf[0..n), n <= PER * NT, keys only
+// (zero pads them and sorts last; equal keys are equal values).  PER
+// consecutive elements per thread in registers: distances below PER inside
+// the thread, up to 32 * PER across the lanes of a wave (DPP, swizzle and
+// bpermute lane moves), 64 * PER and more through buf with barriers.  buf
+// has room for PER * NT keys; all of them are written.
+template <int PER>
 __device__ __forceinline__ void block_sort_desc(uint64_t* buf, int n) {
   const int tid = threadIdx.x;
   uint64_t x[PER];
@@ -757,7 +753,7 @@ __device__ __forceinline__ void block_sort_desc(uint64_t* buf, int n) {
     v = keep_max ? hi : lo;
   };
   #pragma unroll
-  for (int k = 2; k <= PER * NTH; k <<= 1) {
+  for (int k = 2; k <= PER * NT; k <<= 1) {
     #pragma unroll
     for (int j = k >> 1; j > 0; j >>= 1) {
       if (j >= 64 * PER) {
