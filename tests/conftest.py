@@ -27,3 +27,24 @@ def hip():
     assert torch.cuda.is_available(), "GPU test run without a GPU"
     _lib.load()
     return _lib
+
+
+@pytest.fixture
+def new_stream(hip):
+    """Makes streams of their own: torch's come from a pool in turn, and may
+    already hold a buffer of the library's.  Each gives its buffers back."""
+    import ctypes
+    import torch
+    handles = []
+
+    def make():
+        h = ctypes.c_uint64()
+        assert int(torch.cuda.cudart().cudaStreamCreate(ctypes.addressof(h))) == 0
+        handles.append(h)
+        return torch.cuda.ExternalStream(h.value)
+
+    yield make
+    torch.cuda.synchronize()
+    for h in handles:
+        hip.check(hip.load().hi_rocm_sampler_release(h.value))
+        assert int(torch.cuda.cudart().cudaStreamDestroy(h.value)) == 0

@@ -1,5 +1,7 @@
 // Compares hi_amd/csrc/exact_expf.h (host build) with the host glibc expf:
-// every float in [-104, 0] plus every 61st bit pattern elsewhere.
+// every float in [-104, 0] plus every 61st bit pattern elsewhere; the form
+// without branches for x <= 0 (exact_expf_neg, the weights of the
+// whole-distribution draws) on the same values up to -inf.
 #include <math.h>
 #include <pthread.h>
 #include <stdio.h>
@@ -21,7 +23,20 @@ void* work(void* arg) {
     memcpy(&x, &u, 4);
     float a = hi_rocm::exact_expf(x), r = expf(x);
     g_bad[id] += memcmp(&a, &r, 4) != 0;
+    a = hi_rocm::exact_expf_neg(x, hi_rocm::Exp2TabConst{});
+    g_bad[id] += memcmp(&a, &r, 4) != 0;
     g_count[id]++;
+  }
+  for (uint64_t b = 0xC2D00001ull + (uint64_t)id * 61; b <= 0xFF800000ull; b += 61 * kThreads) {
+    const uint32_t u = b + 61 * kThreads > 0xFF800000ull ? 0xFF800000u : (uint32_t)b;  // each ends with -inf
+    float x;
+    memcpy(&x, &u, 4);
+    const float a = hi_rocm::exact_expf_neg(x, hi_rocm::Exp2TabConst{}), r = expf(x);
+    g_bad[id] += memcmp(&a, &r, 4) != 0;
+  }
+  {
+    const float a = hi_rocm::exact_expf_neg(0.f, hi_rocm::Exp2TabConst{});
+    g_bad[id] += a != 1.f;
   }
   // everything else, sampled
   for (uint64_t b = (uint64_t)id * 61; b <= 0xFFFFFFFFull; b += 61 * kThreads) {

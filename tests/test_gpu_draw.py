@@ -143,9 +143,9 @@ GRID = [(9, 262143), (9, 262144), (9, 262145), (12, 262208), (2, 1048577), (40, 
 def test_finish_grid(hip, oracle, B, V, bf16):
     """Two launches (more than 512 workgroups of 4096 logits): nucleus and
     min-p rows through the wide pass, which the path codes show, and
-    temperature-only rows split over workgroups, in units of one chunk (up to
-    768 workgroups) and of four, on both sides of 256 tiles and 256 chunks,
-    rows of any alignment, with and without logprobs."""
+    temperature-only rows split over workgroups (up to 64 rows) or not, on
+    both sides of 256 tiles and 256 chunks, rows of any alignment, with and
+    without logprobs."""
     import torch
     from hi_amd import sampler as S
     n = B * ((V + 4095) // 4096)
@@ -179,8 +179,7 @@ def test_finish_grid(hip, oracle, B, V, bf16):
 @pytest.mark.parametrize("kind", ["levels", "equal", "bf16 values", "both", "own levels", "short", "flat"])
 @pytest.mark.parametrize("B,V", [(16, 151936), (56, 70003)])
 def test_f32_rows_of_few_values(hip, oracle, B, V, kind):
-    """f32 rows whose long lists share values: counted by value in units of
-    one chunk and of four; rows with a unit of other values, which stays
+    """f32 rows whose long lists share values: counted by value; rows with a unit of other values, which stays
     listed beside counted ones; units with levels of their own, too many together for the merge's table
     (their ranks come from the lists after all); rows that share none."""
     import torch
@@ -250,3 +249,29 @@ def test_dense_histories(hip, oracle, B, V, n_hist, bf16):
     assert bad.size == 0, (bad, got[bad], want["tokens"][bad])
     np.testing.assert_allclose(out["logprobs"].cpu().numpy(), want["logprobs"], rtol=1e-5, atol=1e-6)
     assert np.array_equal(out["logprob_ids"].cpu().numpy().view(np.uint32), want["logprob_ids"])
+
+
+@pytest.mark.parametrize("V", [65540, 70001])
+def test_row_kernel_finite_lane_argmax(hip, oracle, new_stream, V):
+    """256 greedy rows by the launchers' finite-lane rule (ties by the
+    bit-reversed lane) in one workgroup each, and the same rows by temperature
+    alone: ties across lanes and tiles, signed zeros, infinities, NaN, rows
+    without a finite logit."""
+    import torch
+    from test_gpu_parity import _finite_lane_rows
+    B = 256
+    x = _finite_lane_rows(V, B, np.random.default_rng(V))
+    u = np.random.default_rng(1).random(B).astype(F32)
+    logits, samples = torch.from_numpy(x).cuda(), torch.from_numpy(u).cuda()
+    out = torch.zeros(B, dtype=torch.int32, device="cuda")
+    st = new_stream()
+    torch.cuda.synchronize()
+    print(f"finite-lane rows V={V}", flush=True)
+    for t in (0.0, 0.8):
+        hip.check(hip.load().hi_rocm_launch_sample_batched_last_token(
+            logits.data_ptr(), out.data_ptr(), samples.data_ptr(), B, 1, V, t, float("inf"), 0, 1, st.cuda_stream))
+        st.synchronize()
+        got = out.cpu().numpy().view(np.uint32).tolist()
+        want = [oracle.argmax_finite_lane(x[b])[0] if t <= 0 else oracle.temp_only_sample(x[b], t, float(u[b]))
+                for b in range(B)]
+        assert got == want, [(b, g, w) for b, (g, w) in enumerate(zip(got, want)) if g != w][:8]

@@ -411,9 +411,9 @@ def _crossing_rows(rng, B, V):
 def test_wide_pass_sums_equal_oracle(hip, oracle, case):
     """The wide pass's normaliser (the vocabulary-order f32 sum of the
     weights, gpu.rs:837) and candidate total (:874) equal the oracle's bit
-    for bit on every top-p row it finishes: this pins the chunk maps, the
-    crossing records and windows, the chain and the rank-order folds, which
-    the tokens alone check only where a sum decides a cut."""
+    for bit on every top-p row it finishes: this pins the tiles' maps, the
+    chain and the rank-order folds, which the tokens alone check only where a
+    sum decides a cut."""
     if case == "crossings":
         rng = np.random.default_rng(77)
         B, V = 24, 151936
@@ -435,8 +435,8 @@ def test_wide_pass_sums_equal_oracle(hip, oracle, case):
 def test_wide_pass_other_seeds(hip, oracle, cfg, seed):
     """C2's and C5's workloads drawn from other seeds: tokens equal to the
     oracle's, every top-p row finished by the wide pass, and its two sums
-    bit-exact.  C2's bf16 rows list thousands of superset runs (their merge
-    input loads before the chain), C5's masked rows fewer (after it)."""
+    bit-exact.  C2's bf16 rows are ranked by value, C5's masked f32 rows from
+    their lists."""
     w = CONFIGS[cfg](seed=seed)
     say(f"config {cfg} seed {seed}: B={w.batch} V={w.vocab}")
     totals, paths = [], []

@@ -3,8 +3,6 @@ restatement of gpu.rs:10725-10762 (host argmax gpu.rs:6406-6435): per-row
 argmax, accepted counts and emitted tokens bit for bit, over drafts that
 are fully accepted, rejected at each position, per-request draft lengths,
 K = 0, ties, NaN and infinities, and a 151,936-token vocabulary."""
-import ctypes
-
 import numpy as np
 import pytest
 
@@ -55,13 +53,6 @@ def test_spec_verify_parity(hip, oracle, B, K, V):
             assert (tt[b, cc[b]:] == 0xffffffff).all(), "write past the emitted tokens"
 
 
-def _stream_of_its_own(torch):
-    """A new stream and its handle (torch's come from a pool)."""
-    handle = ctypes.c_uint64()
-    assert int(torch.cuda.cudart().cudaStreamCreate(ctypes.addressof(handle))) == 0
-    return torch.cuda.ExternalStream(handle.value), handle
-
-
 class _Call:
     """One verification's device arrays and what the oracle says of them."""
 
@@ -92,7 +83,7 @@ class _Call:
 
 
 @pytest.mark.parametrize("V", [1, 8191, 8193, 50257, 70001])
-def test_spec_verify_parts(hip, oracle, V):
+def test_spec_verify_parts(hip, oracle, new_stream, V):
     """Rows split over workgroups (8192 logits each), eagerly and in a capture
     on a stream of no earlier call: maxima on both sides of every part's edge,
     equal maxima in two parts, -inf and NaN rows, and whatever the greedy
@@ -114,7 +105,7 @@ def test_spec_verify_parts(hip, oracle, V):
     d = rng.integers(0, V, (B, K)).astype(np.uint32)
     d[:, 0] = oracle.spec_verify_greedy(x, d, None)[0][:, 0]
     call = _Call(torch, oracle, x, d)
-    s, handle = _stream_of_its_own(torch)
+    s = new_stream()
     torch.cuda.synchronize()
     print(f"spec verify parts V={V}", flush=True)
     graph = torch.cuda.CUDAGraph()
@@ -130,11 +121,10 @@ def test_spec_verify_parts(hip, oracle, V):
         call.launch(hip, s.cuda_stream)
         s.synchronize()
         call.same()
-    del graph, s
-    assert int(torch.cuda.cudart().cudaStreamDestroy(handle.value)) == 0
+    del graph
 
 
-def test_spec_verify_calls_share_nothing(hip, oracle):
+def test_spec_verify_calls_share_nothing(hip, oracle, new_stream):
     """Calls with different outputs at once: two graphs captured on one stream
     and replayed on two others, beside eager calls on the capture stream, each
     checked after every round; releasing the stream's library buffers leaves
@@ -148,8 +138,8 @@ def test_spec_verify_calls_share_nothing(hip, oracle):
         d = x[:, :K].argmax(2).astype(np.uint32)
         d[::3, seed] += 1
         calls.append(_Call(torch, oracle, x, d))
-    s, handle = _stream_of_its_own(torch)
-    others = [torch.cuda.Stream(), torch.cuda.Stream()]
+    s = new_stream()
+    others = [new_stream(), new_stream()]
     for c in calls:  # the kernels' first launches
         c.launch(hip, others[0].cuda_stream)
     torch.cuda.synchronize()
@@ -176,11 +166,10 @@ def test_spec_verify_calls_share_nothing(hip, oracle):
         torch.cuda.synchronize()
         for c in calls:
             c.same()
-    del graphs, s
-    assert int(torch.cuda.cudart().cudaStreamDestroy(handle.value)) == 0
+    del graphs
 
 
-def test_spec_verify_beyond_32_bit_bytes(hip):
+def test_spec_verify_beyond_32_bit_bytes(hip, new_stream):
     """A row of more than 2^32 bytes: the maximum is found wherever it lies,
     and of two equal ones the first."""
     import torch
@@ -188,7 +177,7 @@ def test_spec_verify_beyond_32_bit_bytes(hip):
     V = 2 ** 30 + 5
     x = torch.full((V,), -1.0, device="cuda")
     d, g, t, c = (torch.zeros(2, dtype=torch.int32, device="cuda") for _ in range(4))
-    st = torch.cuda.Stream()
+    st = new_stream()
     for at in ([3], [2 ** 29 - 1, 2 ** 29 + 3], [2 ** 29 + 3], [2 ** 30 - 1, 2 ** 30 + 2], [2 ** 30 + 2], [V - 1]):
         x[at] = 2.0
         torch.cuda.synchronize()

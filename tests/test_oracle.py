@@ -436,7 +436,7 @@ def test_logprobs_match_float64(oracle):
 def test_expf_port_matches_glibc_exhaustively(tmp_path):
     """The weight function the kernels use (hi_amd/csrc/exact_expf.h), built
     for the host, equals glibc expf on every float in [-104, 0] and on a
-    stride sample of the rest."""
+    stride sample of the rest; its form without branches on those up to 0."""
     import subprocess
     src = os.path.join(os.path.dirname(__file__), "native", "expf_port_check.cpp")
     inc = os.path.join(os.path.dirname(os.path.dirname(__file__)), "hi_amd", "csrc")
