@@ -35,14 +35,19 @@ METRIC = "sampled rows/s @B=256 V=129280; µs/step @B=1; % of HBM peak BW"
 PASSES = {
     "row_kernel (B >= 192 f32, no logprobs; C3)": {
         "top-k <= 256 (incl. min-p, penalties, mask)": {"reads": 1, "writes": 0},
-        "other classes, or a fallback (general path, 8192-logit chunks)":
-            {"reads": "1 + 1 of s for top-p / temperature-only / top-k > 1024", "writes": "0, or 1 of s",
-             "l2": "the s re-read"},
+        "greedy": {"reads": 1, "writes": 0},
+        "top-p / min-p without top-k": {
+            "reads": "1 (logits) + 1 of s + 1 of w a fold, and a gather and lookup of w a draw",
+            "writes": "2 (s, w)", "l2": "the s and w re-reads"},
+        "temperature only": {"reads": "1 + 1 of s", "writes": "1 of s", "l2": "the s re-read"},
+        "top-k > 256, or a fallback (general path, 8192-logit chunks)": {
+            "reads": "1 + 1 of s for top-k > 1024", "writes": "0, or 1 of s", "l2": "the s re-read"},
     },
     "select + finish (C1 one launch; C2, C4, C5 two)": {
         "greedy, top-k <= 1024 (C1, C2's greedy half, C4)": {"reads": 1, "writes": 0},
         "top-p without top-k (wide pass; C2, C5)": {
-            "reads": "1 (logits) + 1 (s, finish grid) + the refolded chunks' w (a few per row)",
+            "reads": "1 (logits) + 1 (s, finish grid) + w of the tiles the chain folds itself and of the drawn "
+                     "weight's unit",
             "writes": "2 (s by the select pass, w by the finish grid)", "l2": "the s and w re-reads"},
         "temperature only, top-k > 1024": {"reads": "1 + 1 of s", "writes": "1 of s", "l2": "the s re-read"},
     },

@@ -165,8 +165,10 @@ void carve(hi_rocm::SampleArgs& a, void* ws, const hi_rocm::WorkspaceLayout& L) 
   a.wtot = (float*)(base + L.wtot);
   // Masked rows that do not start on 16 bytes stay with the general scan: the
   // streaming passes send rows of few allowed tokens to their exact fallback
-  // (12 f32 top-k rows of 100,003: 56 us scanned, 134 streamed; 250 rows of
-  // 64,001: 120 and 250).
+  // (scanned and streamed: 12 f32 top-k rows of 100,003 56 and 134 us, 250 rows
+  // of 64,001 120 and 250).  Other rows lie on both sides (f32 rows of 50,257,
+  // half of the tokens allowed: 12 rows greedy 10 and 12, nucleus 104 and 109,
+  // top-k 25 and 18; 64 rows 16 and 13, 117 and 100, 38 and 21).
   if (a.mask != nullptr && !a.vec_ok) a.stream_ok = 0;
   a.chunk = hi_rocm::choose_chunk(a.B, a.V, a.n_lp, a.stream_ok, a.hoff != nullptr);
   a.n_chunks = (a.V + a.chunk - 1) / a.chunk;
