@@ -161,6 +161,7 @@ enum WidePath : uint32_t {
   kRowPathMinp = 8,       // the min-p support finish
   kRowPathLists = 9,      // the candidate lists' finish (finish_core)
   kRowPathGeneral = 10,   // the general path (chunk select and finish)
+  kRowPathAll = 12,       // all sixteen waves (classes other than top-k)
 };
 
 // Batches whose (chunk, row) grid has at most this many workgroups run the

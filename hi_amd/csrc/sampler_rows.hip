@@ -1047,7 +1047,7 @@ __device__ __noinline__ bool row_wide(KernargSampleArgs* ap, int row) {
   }
   if (tid == 0) {
     a.out_tokens[row] = token;
-    a.diag[row] = kRowPathGeneral;
+    a.diag[row] = kRowPathAll;
   }
   return true;
 }

@@ -232,7 +232,7 @@ class Sampler:
 
 WIDE_PATHS = {0: "other", 1: "wide", 2: "no-stats", 3: "chunk-full", 4: "total", 5: "merge-full",
               6: "no-cutoff", 7: "draw-fail", 8: "row-minp", 9: "row-lists", 10: "row-general",
-              11: "long-list"}
+              11: "long-list", 12: "row-all"}
 
 
 def debug_wide_paths(smp: "Sampler", batch: int, vocab: int,

@@ -275,3 +275,34 @@ def test_row_kernel_finite_lane_argmax(hip, oracle, new_stream, V):
         want = [oracle.argmax_finite_lane(x[b])[0] if t <= 0 else oracle.temp_only_sample(x[b], t, float(u[b]))
                 for b in range(B)]
         assert got == want, [(b, g, w) for b, (g, w) in enumerate(zip(got, want)) if g != w][:8]
+
+
+@pytest.mark.parametrize("with_mask", [False, True])
+def test_row_kernel_path_of_other_classes(hip, with_mask):
+    """Which rows of a 256-row batch all waves finish: every class but top-k,
+    unless the history is too long for their table or no logit is finite."""
+    import torch
+    from hi_amd import sampler as S
+    B, V = 256, 65540
+    rng = np.random.default_rng(3)
+    x = _rows("spiked", B, V, 5)
+    x[3, :] = -np.inf
+    p = _params(B)
+    p["top_k"][4::5] = 40
+    p["temperature"][10::20] = 0.0
+    n = np.where(np.arange(B) == 21, 3500, 50)
+    off = np.concatenate([[0], np.cumsum(n)]).astype(np.uint32)
+    ids = rng.integers(0, V, off[-1]).astype(np.uint32)
+    mask = np.full((B, (V + 31) // 32), 0xffffffff, np.uint32) if with_mask else None
+    i32 = lambda a: torch.from_numpy(a.view(np.int32)).cuda()  # noqa: E731
+    smp = S.Sampler(B, V)
+    print(f"row kernel paths mask={with_mask}", flush=True)
+    smp.sample(torch.from_numpy(x).cuda(), S.params_to_device(p), torch.full((B,), 0.5, device="cuda"), i32(off),
+               i32(ids), i32(np.ones_like(ids)), None if mask is None else i32(mask))
+    torch.cuda.synchronize()
+    names = np.array([S.WIDE_PATHS.get(int(c) & 0xff) for c in S.debug_wide_paths(smp, B, V)])
+    topk = (p["top_k"] > 0) & (p["temperature"] > 0)
+    left = np.isin(np.arange(B), [21] if with_mask else [3, 21])  # (masked rows without a finite logit give eos)
+    assert set(names[~topk & ~left]) == {"row-all"}, names
+    assert set(names[left]) == {"row-general"}, names[left]
+    assert "row-all" not in names[topk]
