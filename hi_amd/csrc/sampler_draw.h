@@ -514,16 +514,18 @@ __device__ __forceinline__ void draw_descend(DrawLds<NTH>& D, const DrawRow& r, 
     });
     __syncthreads();
     if (tid < 64) {
-      // from bin 2047 down, 32 bins a lane (rolled: the loads of all 32 in
-      // flight made this rare path the kernels' register peak, 256 + 12
-      // instead of 214)
+      // from bin 2047 down, 32 bins a lane (rolled for four waves: the loads
+      // of all 32 in flight made this rare path those kernels' register peak,
+      // 256 + 12 instead of 214; sixteen waves have 128 either way, and the
+      // mixed rows of the row kernel take 0.7% longer rolled)
+      constexpr int kRolled = NTH >= 1024 ? 32 : 4, kRolled1 = NTH >= 1024 ? 32 : 1;
       uint32_t c = 0u;
-      #pragma unroll 4
+      #pragma unroll kRolled
       for (int k = 0; k < 32; ++k) c += D.hist[draw_slot((uint32_t)(2047 - 32 * lane - k))];
       uint32_t cum = wave_incl_scan_u32(c) - c;
       int low = -1, first = -1;  // the last bin that still fits; the first nonempty one
       bool stop = false;
-      #pragma unroll 1
+      #pragma unroll kRolled1
       for (int k = 0; k < 32 && !stop; ++k) {
         const int b = 2047 - 32 * lane - k;
         const uint32_t h = D.hist[draw_slot((uint32_t)b)];
